@@ -7,7 +7,7 @@
  * int status (NF4_OK == 0).  The caller allocates every output and workspace, and apart from
  * one entry point the library owns no device memory and keeps no state between calls, so it is
  * reentrant and thread-safe.  The exception is nf4_linear_dx_noalloc (for callers that cannot
- * allocate): its split-K partials live in a 64 MiB device array that the library holds on every
+ * allocate): its workspace is a 64 MiB device array that the library holds on every
  * GPU it runs on until the process ends, and calls of it that overlap on one GPU race.
  *
  * Weight format (bitsandbytes 0.50.2 QuantState, as read by the reference at
@@ -138,7 +138,11 @@ int nf4_dequant_table(const void *dev_table, int nw, int64_t blocks, int out_dty
  * Replaces: F.linear(x, dequantize_nf4(W), bias) in NF4Linear.forward (nf4.py:84-91); the
  *           addmm / mm projection GEMMs of FusedDecoderLayer.forward with the LoRA terms
  *           (layer.py:871-878, 893, 914, 929); RecomputedMLP's forward GEMMs (mlp.py:47-54).
- * workspace may be NULL when nf4_linear_fwd_workspace() returns 0 for the same arguments. */
+ * workspace may be NULL when nf4_linear_fwd_workspace() returns 0 for the same arguments.  From
+ * 512 tokens on, where it is faster, the call dequantizes the stacked weight into the
+ * workspace (2 bytes per element, rows padded to 128) and multiplies it there: 16-byte aligned
+ * outputs with a row stride of a multiple of 8 and a 256-byte aligned workspace take that route,
+ * others the fused one, for which the same workspace suffices. */
 int nf4_linear_fwd(const void *x, int64_t m, int64_t ldx,
                    const nf4_weight *ws, int nw, const void *bias,
                    const nf4_lora *loras, int nlora,
@@ -160,13 +164,13 @@ size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int nw, int dtyp
 
 /* nf4_linear_dx without a workspace argument: it allocates nothing, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid allocation).  No counterpart in the reference.  Split-K partials go to one static
+ * forbid allocation).  No counterpart in the reference.  Its workspace is one static
  * device array of NF4_STATIC_SCRATCH_BYTES per GPU, set up when the library's code loads on a
  * device and held until the process ends; its address is looked up on the first call on each
- * device (make that first call outside graph capture).  The tiling is nf4_linear_dx's, chosen
- * among the plans whose partials fit the array (plans with no split need none), so every size
+ * device (make that first call outside graph capture).  The plan is nf4_linear_dx's where its
+ * workspace fits the array, else the best fused tiling whose partials do, so every size
  * is accepted; the result equals nf4_linear_dx's bit for bit whenever its plan fits.  The
- * array keeps the last call's partials; calls that overlap on one GPU (other streams or
+ * array keeps the last call's contents; calls that overlap on one GPU (other streams or
  * threads) share it and race.  The stream must belong to the current device. */
 #define NF4_STATIC_SCRATCH_BYTES (64u << 20)
 int nf4_linear_dx_noalloc(const void *dy, int64_t m, int64_t lddy,

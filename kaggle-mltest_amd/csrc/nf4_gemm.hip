@@ -37,7 +37,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "nf4_common.h"
+#include "nf4_dense.h"
 
 namespace {
 
@@ -2599,6 +2599,7 @@ struct Plan {
     int rows_g = 0;  // row-streaming path: row groups per workgroup
     int dks = 0;     // skinny path: super-step depth (128 or 256)
     int fx = 0;      // skinny path: LoRA down-projections computed in the launch
+    double cost = 0; // tiled paths: the model's time
 
     int64_t blocks() const { return tail_start + (tiles - tail_start) * splits; }
 };
@@ -2714,7 +2715,7 @@ Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_spl
                 if (best.splits == 0 || c < best_cost) {
                     best = Plan{cfg, cfg == 0 ? 256 : 128, cfg == 0 ? 256 : 128, s, tiles, 0,
                                 s > 1 ? ts : tiles};
-                    best_cost = c;
+                    best_cost = best.cost = c;
                 }
             }
         }
@@ -2732,7 +2733,7 @@ Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_spl
             const double c = head + plan_cost(cfg, tail, mt1, tail, 1, steps, m) + kLaunchGap;
             if (c < best_cost) {
                 best = Plan{cfg, 128, 128, 1, tail, 0, tail, hp};
-                best_cost = c;
+                best_cost = best.cost = c;
             }
         }
     }
@@ -3179,24 +3180,134 @@ int64_t dx_tail_col0(const Plan &p, int64_t m) {
     return (p.tail_start / mt) * p.bp;
 }
 
+// ------------------------------------------------- dequantized once, multiplied densely
+//
+// From a thousand tokens or so on, dequantizing every weight tile again for each 256 tokens costs
+// more than writing the 16-bit weight to a workspace once (2.5 bytes per element at ~6.6 TB/s)
+// and multiplying it with a kernel free of dequantization (nf4_dense.hip).  Measured at M = 8192
+// (7B, bf16): gate|up forward 2109 -> 1799 us, its input gradient 2190 -> 1835, down 1123 -> 902;
+// at M = 512 the same products are 156 fused against 195.
+
+struct DenseRoute {
+    bool use;
+    DensePlan plan;
+    size_t weight_bytes;   // the dequantized weight, at the start of the workspace
+    size_t bytes;          // with the split's partials
+};
+
+// The time of a fused plan in a layer's sequence of products, from the model's: plan_cost was
+// fitted to each launch by itself at M = 2048; over M = 384 .. 8192 these factors bring it to
+// 5.9 % rms (a second round of 128x128 tiles costs 9 us more than it says, and every
+// further segment of an input gradient, whose pipeline restarts, 2.4 us).
+double fused_time(const Plan &p, int64_t small_tiles, int extra_segs) {
+    const double busy = small_tiles < kCUs ? double(small_tiles) / kCUs : 1.0;
+    const double f = p.head_ptiles > 0 ? 0.876 : p.cfg == 0 ? 0.784 : p.cfg == 1 ? 0.907 : 0.846 + 0.206 * busy;
+    const bool rounds = p.cfg == 1 && p.splits == 1 && p.head_ptiles == 0 && small_tiles > kCUs;
+    return p.cost * f + (rounds ? 9.1 : 0.0) + 2.4 * extra_segs;
+}
+
+// Taken where it is 4 % faster by the two models (10 % with a split reduction, whose partials
+// come on top of the weight in the workspace): of 308 measured (projection, direction, M, dtype)
+// points no fused one faster by more than 1 % is given up.  Below 512 tokens the
+// dequantization alone costs what the fused kernels need.
+DenseRoute dense_route(int64_t P, int64_t m, int64_t R, double dequant_us, double fused_us) {
+    DenseRoute r{};
+    if (m < 512 || (P + 127) * R >= (int64_t(1) << 30)) return r;
+    r.plan = dense_plan(P, m, R);
+    r.use = r.plan.cost + dequant_us < (r.plan.splits > 1 ? 0.90 : 0.96) * fused_us;
+    r.weight_bytes = static_cast<size_t>((P + 127) / 128) * 256 * R;  // strips (nf4_dense.h)
+    r.bytes = r.weight_bytes + (r.plan.splits > 1 ? static_cast<size_t>(r.plan.splits) * m * P * 4 : 0);
+    return r;
+}
+
+DenseRoute dense_route_fwd(int64_t m, const nf4_weight *ws, int nw, const Plan &p) {
+    if (p.cfg != 0 && p.cfg != 1 && p.cfg != 3) return DenseRoute{};
+    int64_t n = 0, small = 0;
+    for (int i = 0; i < nw; ++i) {
+        n += ws[i].rows;
+        small += (ws[i].rows + 127) / 128 * ((m + 127) / 128);
+    }
+    if (ws[0].cols % 128 != 0) return DenseRoute{};
+    return dense_route(n, m, ws[0].cols, 9.8 + 2.52 * double(n) * double(ws[0].cols) / 4.78e6,
+                       fused_time(p, small, 0));
+}
+
+// (the strips take whole 64-row, 128-column pieces of every segment)
+DenseRoute dense_route_dx(int64_t m, const nf4_weight *ws, int nw, const Plan &p) {
+    const int64_t K = ws[0].cols;
+    int64_t n = 0;
+    for (int i = 0; i < nw; ++i) {
+        if (ws[i].rows % 64 != 0) return DenseRoute{};
+        n += ws[i].rows;
+    }
+    if (n == 0 || K % 128 != 0) return DenseRoute{};
+    return dense_route(K, m, n, 12.9 + 2.52 * double(n) * double(K) / 5.37e6,
+                       fused_time(p, (K + 127) / 128 * ((m + 127) / 128), nw - 1));
+}
+
+// The second launch of the dense route and, of a split plan, the reduction: g holds the call.
+int launch_dense(GemmArgs &g, const DenseRoute &r, int nw, bool dx, void *workspace, int dtype, hipStream_t s) {
+    DenseArgs a = {};
+    a.w = static_cast<const uint16_t *>(workspace);
+    a.act = g.act;
+    a.ld_act = g.ld_act;
+    a.P = g.n_out;
+    a.M = g.M;
+    a.R = g.act_cols;
+    a.out = static_cast<uint16_t *>(g.out);
+    a.ld_out = g.ld_out;
+    a.bias = r.plan.splits > 1 ? nullptr : g.bias;  // (a split plan's reduction adds it)
+    for (int i = 0; i < nw; ++i) {
+        const LoraDev &l = g.lora[i];
+        if (!l.has) continue;
+        DenseSlab &sl = a.slab[a.nslab++];
+        sl.rank = l.rank;
+        sl.scale = dx ? 1.0f : l.scale;  // (da holds the scale)
+        if (dx) {
+            sl.l = l.a, sl.lp = 1, sl.lr = g.K, sl.vec_l = 0;
+            sl.t = l.da, sl.vec_t = l.vec;
+            sl.p_lo = 0, sl.p_hi = g.K;
+        } else {
+            sl.l = l.b, sl.lp = l.rank, sl.lr = 1, sl.vec_l = l.vec;
+            sl.t = l.t, sl.vec_t = l.vec;
+            sl.p_lo = g.seg_off[i], sl.p_hi = g.seg_off[i] + g.w[i].rows;
+        }
+    }
+    a.partial = reinterpret_cast<float *>(static_cast<char *>(workspace) + r.weight_bytes);
+    const int st = dense_gemm(a, r.plan, dtype, s);
+    if (st != NF4_OK || r.plan.splits <= 1) return st;
+    g.partial = a.partial;
+    g.tail_col0 = 0;
+    g.tail_cols = g.n_out;
+    return dtype == NF4_BF16 ? launch_reduce<NF4_BF16>(g, r.plan.splits, s)
+                             : launch_reduce<NF4_F16>(g, r.plan.splits, s);
+}
+
 }  // namespace
 
 extern "C" size_t nf4_linear_fwd_workspace(int64_t m, const nf4_weight *ws, int nw, int dtype) {
     (void)dtype;
     if (!ws || nw < 1 || nw > kMaxSeg || m <= 0) return 0;
     const Plan p = plan_fwd(m, ws, nw);
-    if (p.splits <= 1) return 0;
-    int64_t n = 0;
-    for (int i = 0; i < nw; ++i) n += ws[i].rows;
-    return static_cast<size_t>(p.splits) * m * (n - fwd_tail_col0(p, m, ws, nw)) * sizeof(float);
+    const DenseRoute dense = dense_route_fwd(m, ws, nw, p);
+    size_t need = dense.use ? dense.bytes : 0;
+    if (p.splits > 1) {  // (also where the dense route is taken: a call that it does not fit)
+        int64_t n = 0;
+        for (int i = 0; i < nw; ++i) n += ws[i].rows;
+        const size_t fused = static_cast<size_t>(p.splits) * m * (n - fwd_tail_col0(p, m, ws, nw)) * sizeof(float);
+        if (fused > need) need = fused;
+    }
+    return need;
 }
 
 extern "C" size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int nw, int dtype) {
     (void)dtype;
     if (!ws || nw < 1 || nw > kMaxSeg || m <= 0) return 0;
     const Plan p = plan_dx(m, ws, nw);
-    if (p.splits <= 1) return 0;
-    return static_cast<size_t>(p.splits) * m * (ws[0].cols - dx_tail_col0(p, m)) * sizeof(float);
+    const DenseRoute dense = dense_route_dx(m, ws, nw, p);
+    const size_t fused =
+        p.splits > 1 ? static_cast<size_t>(p.splits) * m * (ws[0].cols - dx_tail_col0(p, m)) * sizeof(float) : 0;
+    return dense.use && dense.bytes > fused ? dense.bytes : fused;
 }
 
 extern "C" int nf4_linear_fwd_tiled(const void *x, int64_t m, int64_t ldx, const nf4_weight *ws,
@@ -3302,6 +3413,14 @@ extern "C" int nf4_linear_fwd_tiled(const void *x, int64_t m, int64_t ldx, const
         }
         return status_of(hipGetLastError());
     }
+    if (tile < 0 && g.vec16_out && aligned(workspace, 256)) {
+        const DenseRoute dense = dense_route_fwd(m, ws, nw, p);
+        if (dense.use && workspace && workspace_bytes >= dense.bytes) {
+            hipStream_t s = static_cast<hipStream_t>(stream);
+            st = dequant_strips(ws, nw, false, workspace, dtype, s);
+            return st != NF4_OK ? st : launch_dense(g, dense, nw, false, workspace, dtype, s);
+        }
+    }
     g.splits = p.splits;
     // reduction steps per split: BR-deep steps, or the skinny path's super-steps
     const int64_t unit = p.cfg == 7 ? p.dks : BR;
@@ -3385,6 +3504,14 @@ int linear_dx_impl(const void *dy, int64_t m, int64_t lddy, const nf4_weight *ws
     g.accumulate = accumulate != 0;
     g.vec_out = aligned(dx, 8) && lddx % 4 == 0;
     g.vec16_out = aligned(dx, 16) && lddx % 8 == 0;
+    if (tile < 0 && g.vec16_out && !accumulate && aligned(workspace, 256)) {
+        const DenseRoute dense = dense_route_dx(m, ws, nw, plan_dx(m, ws, nw));
+        if (dense.use && workspace && workspace_bytes >= dense.bytes) {
+            hipStream_t s = static_cast<hipStream_t>(stream);
+            st = dequant_strips(ws, nw, true, workspace, dtype, s);
+            return st != NF4_OK ? st : launch_dense(g, dense, nw, true, workspace, dtype, s);
+        }
+    }
     const Plan p = plan_dx(m, ws, nw, tile, splits, ws_cap);
     if (p.splits == 0) return NF4_ERR_ARG;
     g.splits = p.splits;
