@@ -2695,8 +2695,8 @@ double plan_cost(int cfg, int64_t tiles, int64_t mt, int64_t tail_start, int spl
 
 // `ws_cap` >= 0 (input-gradient plans only, `out_cols` = K): leave out split plans whose fp32
 // partials, splits x M x (columns from the tail's first p tile to K), exceed ws_cap bytes.
-Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_splits = kMaxSplits,
-               int64_t out_cols = 0, int64_t ws_cap = -1) {
+Plan search_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_splits,
+                 int64_t out_cols, int64_t ws_cap) {
     Plan best{};
     double best_cost = 0.0;
     for (int cfg : {0, 1, 3}) {
@@ -2738,6 +2738,32 @@ Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_spl
         }
     }
     return best;
+}
+
+// search_plan's result for the same sizes: a plan is a pure function of them, a program repeats
+// a few dozen of them, and a call asks two or three times (its workspace size, the launch, the
+// dense route), 15-30 us of host time each where the splits are searched.  One table of the
+// last plan per slot and thread; nothing in it refers to a tensor.
+Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_splits = kMaxSplits,
+               int64_t out_cols = 0, int64_t ws_cap = -1) {
+    struct Slot {
+        int64_t key[7];
+        Plan plan;
+        bool used;
+    };
+    static thread_local Slot slots[64];
+    const int64_t key[7] = {m, big, small, steps, max_splits, out_cols, ws_cap};
+    uint64_t h = 0;
+    for (const int64_t v : key) h = (h ^ static_cast<uint64_t>(v)) * 0x9E3779B97F4A7C15ull;
+    Slot &sl = slots[h >> 58];
+    bool same = sl.used;
+    for (int i = 0; i < 7; ++i) same = same && sl.key[i] == key[i];
+    if (!same) {
+        sl.plan = search_plan(m, big, small, steps, max_splits, out_cols, ws_cap);
+        for (int i = 0; i < 7; ++i) sl.key[i] = key[i];
+        sl.used = true;
+    }
+    return sl.plan;
 }
 
 Plan plan_gemv(int64_t m, const nf4_weight *ws, int nw) {

@@ -180,8 +180,14 @@ def check(status: int, what: str) -> None:
     raise cls(f"{what}: {text} (status {status})")
 
 
+# the handle alone, without building a torch.cuda.Stream around it (0.2 us instead of 2)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """The handle of torch's current stream on `t`'s device (what every launch goes to)."""
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
