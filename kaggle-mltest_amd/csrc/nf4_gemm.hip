@@ -1502,9 +1502,9 @@ void decode_kernel(const GemmArgs a) {
     if (lo.has && wave == NW - 1) {
         for (int k0 = 0; k0 < lo.rank; k0 += 32) {
             const int lim = lo.rank - (k0 + 8 * g);
-            const u32x4_t fa = (row < w.rows && lim > 0) ? gather8(lo.b + row * lo.rank + k0 + 8 * g, 1, lim)
+            const u32x4_t fa = (row < w.rows && lim > 0) ? lora_row8(lo.b + row * lo.rank + k0 + 8 * g, lim, lo.vec)
                                                          : (u32x4_t){0u, 0u, 0u, 0u};
-            const u32x4_t fb = (r < a.M && lim > 0) ? gather8(lo.t + r * lo.rank + k0 + 8 * g, 1, lim)
+            const u32x4_t fb = (r < a.M && lim > 0) ? lora_row8(lo.t + r * lo.rank + k0 + 8 * g, lim, lo.vec)
                                                     : (u32x4_t){0u, 0u, 0u, 0u};
             acc = mfma16<DT>(fa, fb, acc);
         }
@@ -1718,12 +1718,12 @@ __global__ __launch_bounds__(RT * KP * 64) void skinny_kernel(const GemmArgs a) 
     if (lo.has && !fx && kp == 0 && split == 0) {
         for (int k0 = 0; k0 < lo.rank; k0 += 32) {
             const int lim = lo.rank - (k0 + 8 * g);
-            const u32x4_t fa = (row < w.rows && lim > 0) ? gather8(lo.b + row * lo.rank + k0 + 8 * g, 1, lim)
+            const u32x4_t fa = (row < w.rows && lim > 0) ? lora_row8(lo.b + row * lo.rank + k0 + 8 * g, lim, lo.vec)
                                                          : (u32x4_t){0u, 0u, 0u, 0u};
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 const int64_t m = 16 * mt + r;
-                const u32x4_t fb = (m < a.M && lim > 0) ? gather8(lo.t + m * lo.rank + k0 + 8 * g, 1, lim)
+                const u32x4_t fb = (m < a.M && lim > 0) ? lora_row8(lo.t + m * lo.rank + k0 + 8 * g, lim, lo.vec)
                                                         : (u32x4_t){0u, 0u, 0u, 0u};
                 acc[mt] = mfma16<DT>(fa, fb, acc[mt]);
             }
@@ -1832,7 +1832,7 @@ __global__ __launch_bounds__(RT * KP * 64) void skinny_kernel(const GemmArgs a) 
             // the slab: Y_seg += scale * T B^T, k over the 16 (zero-padded) ranks
             if (kp == 0) {
                 const int lim = lo.rank - 8 * g;
-                const u32x4_t fa = (row < w.rows && lim > 0) ? gather8(lo.b + row * lo.rank + 8 * g, 1, lim)
+                const u32x4_t fa = (row < w.rows && lim > 0) ? lora_row8(lo.b + row * lo.rank + 8 * g, lim, lo.vec)
                                                              : (u32x4_t){0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
@@ -1852,6 +1852,175 @@ __global__ __launch_bounds__(RT * KP * 64) void skinny_kernel(const GemmArgs a) 
                 epilogue16<DT>(a, acc[mt], p0 + 16 * rt + 4 * g, w.rows, a.seg_off[seg], 16 * mt + r);
         }
     }
+}
+
+// ------------------------------------------- skinny forward path, 17-64 tokens, tall weights
+//
+// The skinny path on v_mfma_f32_32x32x16 for 17 to 64 tokens (MT groups of 32): A = 32 weight
+// rows, lane l row l % 32 and k values 64 (l / 32) .. + 63 of a 128-deep super-step, one absmax
+// block and so one table per 64 elements; k-substep j its 8 values 8 j .. (nibble-plane order,
+// the activations staged in it).  Bound by VALU + MFMA issue: on the 16-row kernel the 7B
+// gate|up at M = 64 issued 5.85 VALU instructions per element (a table per 32 elements, the
+// activations staged again for every 128 rows) and read four fragments per A fragment; here 4.0 and two.
+// A workgroup of 5 x 2 waves owns 160 rows: the 1184 row tiles of the 7B gate|up are 237
+// workgroups, one round of the chip, where 128-row workgroups took two with a split
+// reduction.  That product at M = 64: 61 -> 46 us, at 32: 44 -> 38.  (Before the fragments were read
+// ahead 50 us; then three k-parts, 15 waves, 50.6, four or two row tiles, or a split
+// reduction, 61 us and more.)
+constexpr int kTallRt = 5, kTallKp = 2;
+
+template <int DT, int MT>
+__global__ __launch_bounds__(kTallRt *kTallKp * 64) void skinny32_kernel(const GemmArgs a) {
+    constexpr int RT = kTallRt, KP = kTallKp, NT = RT * KP * 64;
+    constexpr int WS = 2, MP = 32 * MT, XROW = 256, SS = 128;
+    constexpr int XSTG = KP * MP * XROW, NCHUNK = KP * MP * 16;
+    constexpr int CH = (NCHUNK + NT - 1) / NT;  // staged 16-byte chunks per thread
+    static_assert((KP - 1) * RT * MT * 4096 <= 2 * XSTG, "the k-part sums fit in the stages");
+    __shared__ __attribute__((aligned(16))) uint8_t s_x[2 * XSTG];  // [2][KP][MP] rows of 256 bytes
+    __shared__ float s_code2[256];
+
+    const int64_t tile = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x));
+    const int seg = seg_of_tile(a, a.map[0], tile);
+    const int64_t p0 = uniform64((tile - a.map[0].tile_start[seg]) * (32 * RT));
+    const DevWeight w = a.w[seg];
+    const int64_t K = a.K;
+    const int ss = static_cast<int>(K / SS);
+    const int per = (ss + KP - 1) / KP;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int rt = wave % RT, kp = wave / RT;
+    const int my0 = kp * per;
+    const int my_n = ss - my0 < per ? (ss - my0 > 0 ? ss - my0 : 0) : per;
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+
+    for (int i = threadIdx.x; i < 256; i += NT) s_code2[i] = code2_entry(w, i);
+    float code_r[16];
+    load_code_sgpr(w.code, code_r);
+
+    const WeightRsrc wr = weight_rsrc(w);
+    const int64_t row = p0 + 32 * rt + r;
+    const int wpk = static_cast<int>(row * (K >> 1) + 32 * h);
+    const int wblk = static_cast<int>(row * (K >> wr.bs_shift));
+    const int last = my_n > 0 ? my0 + my_n - 1 : 0;
+    struct WStage {
+        u32x4_t raw[2];
+        AbsIn abs;
+    };
+    auto wload = [&](WStage &s, int v) {  // past the part's end: its last super-step again
+        const int st = my0 + v < last ? my0 + v : last;
+        s.raw[0] = bload16(wr.packed, wpk + st * (SS / 2));
+        s.raw[1] = bload16(wr.packed, wpk + st * (SS / 2) + 16);
+        s.abs = absmax_bload(wr, wblk + ((st * SS + 64 * h) >> wr.bs_shift));
+    };
+    // chunk c of a stage: k-part c / (16 MP), token (c / 16) % MP, 16-byte column c % 16
+    // (super-steps past K read the next row's bytes or zero: never used)
+    const int64_t mrows = a.M < MP ? a.M : MP;
+    const rsrc_t xr = make_rsrc(a.act, ((mrows - 1) * a.ld_act + a.act_cols) * 2);
+    const int ldb = static_cast<int>(a.ld_act) * 2;
+    u32x4_t xs[CH];
+    auto xload = [&](int rd) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int c = static_cast<int>(threadIdx.x) + i * NT;
+            if (NCHUNK % NT != 0 && c >= NCHUNK) continue;
+            xs[i] = bload16(xr, (c / 16) % MP * ldb + (c / (16 * MP) * per + rd) * XROW + c % 16 * 16);
+        }
+    };
+    auto xstore = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int c = static_cast<int>(threadIdx.x) + i * NT;
+            if (NCHUNK % NT != 0 && c >= NCHUNK) continue;
+            *reinterpret_cast<u32x4_t *>(s_x + b * XSTG + c / 16 * XROW + (((c % 16) ^ (c / 16 % 16)) << 4)) =
+                plane_order(xs[i]);
+        }
+    };
+
+    float16_t acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = (float16_t){};
+    const LoraDev &lo = a.lora[seg];
+    if (lo.has && kp == 0) {
+        for (int k0 = 0; k0 < lo.rank; k0 += 16) {
+            const int lim = lo.rank - (k0 + 8 * h);
+            const u32x4_t fa = (row < w.rows && lim > 0) ? lora_row8(lo.b + row * lo.rank + k0 + 8 * h, lim, lo.vec)
+                                                         : (u32x4_t){0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int64_t m = 32 * mt + r;
+                const u32x4_t fb = (m < a.M && lim > 0) ? lora_row8(lo.t + m * lo.rank + k0 + 8 * h, lim, lo.vec)
+                                                        : (u32x4_t){0u, 0u, 0u, 0u};
+                acc[mt] = mfma32<DT>(fa, fb, acc[mt]);
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt] *= lo.scale;
+    }
+
+    WStage wst[WS];
+#pragma unroll
+    for (int b = 0; b < WS; ++b) wload(wst[b], b);
+    xload(0);
+    xstore(0);
+    __syncthreads();  // code2 table, activation stage 0
+
+    int xo[8];  // this lane's fragment chunk of k-substep j in a token row
+#pragma unroll
+    for (int j = 0; j < 8; ++j) xo[j] = r * XROW + (((8 * h + j) ^ (r & 15)) << 4);
+    auto compute = [&](const WStage &s, int b) {
+        const Nf4Table tb = make_table<DT>(code_r, absmax_val(w, s.abs, s_code2));
+        const uint8_t *xb = s_x + b * XSTG + kp * MP * XROW;
+        u32x4_t fb[2][MT];  // fragments, read one k-substep ahead (48.4 -> 45.8 us)
+        auto frag = [&](int j) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                fb[j & 1][mt] = *reinterpret_cast<const u32x4_t *>(xb + mt * 32 * XROW + xo[j]);
+        };
+        frag(0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const u32x4_t &raw = s.raw[j / 4];
+            const uint32_t wd = j % 4 == 0 ? raw.x : j % 4 == 1 ? raw.y : j % 4 == 2 ? raw.z : raw.w;
+            if (j < 7) frag(j + 1);
+            const u32x4_t fa = lookup8_planes(tb, wd);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma32<DT>(fa, fb[j & 1][mt], acc[mt]);
+        }
+    };
+    auto round = [&](WStage &s, int rd) {
+        if (rd + 1 < per) xload(rd + 1);
+        if (rd < my_n) compute(s, rd & 1);
+        wload(s, rd + WS);
+        if (rd + 1 < per) xstore((rd + 1) & 1);
+        __syncthreads();
+    };
+    int rd = 0;
+    for (; rd + WS <= per; rd += WS) {
+#pragma unroll
+        for (int b = 0; b < WS; ++b) round(wst[b], rd + b);
+    }
+    if (rd < per) round(wst[0], rd);
+
+    // the k-parts' sums in order, through the stages
+    float4_t *red = reinterpret_cast<float4_t *>(s_x);
+    if (kp > 0) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                red[((((kp - 1) * RT + rt) * MT + mt) * 4 + q) * 64 + lane] =
+                    (float4_t){acc[mt][4 * q], acc[mt][4 * q + 1], acc[mt][4 * q + 2], acc[mt][4 * q + 3]};
+    }
+    __syncthreads();
+    if (kp > 0) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float4_t v = {acc[mt][4 * q], acc[mt][4 * q + 1], acc[mt][4 * q + 2], acc[mt][4 * q + 3]};
+#pragma unroll
+            for (int k = 1; k < KP; ++k) v += red[((((k - 1) * RT + rt) * MT + mt) * 4 + q) * 64 + lane];
+            epilogue16<DT>(a, v, p0 + 32 * rt + 8 * q + 4 * h, w.rows, a.seg_off[seg], 32 * mt + r);
+        }
 }
 
 // ------------------------------------------------------------------- small-M forward path
@@ -2586,7 +2755,7 @@ struct Plan {
     int cfg;       // 0: 256x256 tile / 8 waves, 1: 128x128 tile / 4 waves, 3: 128x128 tile /
                    // two k-groups of 4 waves, 2: small-M path,
                    // 4: decode path (M <= 16), 6: row streaming (M <= 2), 7: skinny path
-                   // (2 < M <= 64)
+                   // (2 < M <= 64), 8: its 32-row kernel (16 < M <= 64, tall weights)
     int bp, bm;
     int splits;    // reduction splits of the tail tiles
     int64_t tiles;
@@ -2998,6 +3167,16 @@ bool skinny_ok(int64_t m, const nf4_weight *ws, int nw, int xa_rank) {
     return t < decode_cost(m, ws, nw) + (xa_rank > 0 ? xa_launch_cost(ws[0].cols) : 0.0);
 }
 
+// The 32-row skinny plan and its time: rounds of 160-row workgroups over the CUs, each step of
+// its two k-parts 2.85 us at 33-64 tokens and 2.3 at 17-32 (7B gate|up: 45.8 and 38.2 us).
+Plan plan_skinny32(int64_t m, const nf4_weight *ws, int nw, double *cost) {
+    int64_t wgs = 0;
+    for (int i = 0; i < nw; ++i) wgs += (ws[i].rows + 32 * kTallRt - 1) / (32 * kTallRt);
+    const int64_t per = (ws[0].cols / DK + kTallKp - 1) / kTallKp;
+    *cost = 6.0 + double((wgs + kCUs - 1) / kCUs) * double(per) * (m > 32 ? 2.85 : 2.3);
+    return Plan{8, 32 * kTallRt, m > 32 ? 64 : 32, 1, wgs, 0, wgs};
+}
+
 // rows_allowed: the row-streaming path's operand alignment holds (LoRA T and B read as dwords).
 // xa_rank: the call's LoRA adapters ask for their down-projections (rank of the largest), which
 // only moves the choice between the skinny and decode paths (neither needs a workspace).
@@ -3005,8 +3184,11 @@ Plan plan_fwd(int64_t m, const nf4_weight *ws, int nw, int tile = -1, int splits
               bool rows_allowed = true, int xa_rank = 0) {
     if (tile < 0 && rows_allowed && rows_ok(m, ws, nw)) return plan_rows(m, ws, nw);
     if (tile < 0 && skinny_ok(m, ws, nw, xa_rank)) {
-        double t = 0;
-        return choose_skinny(m, ws, nw, xa_rank, &t);
+        double t = 0, t32 = 1e30;
+        const Plan p = choose_skinny(m, ws, nw, xa_rank, &t);
+        if (m <= 16) return p;
+        const Plan p32 = plan_skinny32(m, ws, nw, &t32);
+        return t32 + (xa_rank > 0 ? xa_launch_cost(ws[0].cols) : 0.0) < 0.95 * t ? p32 : p;
     }
     if (tile < 0 && m <= kDecodeMaxM && ws[0].cols % DK == 0) return plan_decode(ws, nw);
     if (tile < 0 && m <= kGemvMaxM) return plan_gemv(m, ws, nw);
@@ -3082,6 +3264,12 @@ bool launch_skinny(const GemmArgs &g, const Plan &p, hipStream_t st) {
 template <int DT>
 int launch_fwd(const GemmArgs &g, const Plan &p, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>(p.blocks()));
+    if (p.cfg == 8) {
+        const dim3 block(kTallRt * kTallKp * 64);
+        if (p.bm == 32) hipLaunchKernelGGL((skinny32_kernel<DT, 1>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((skinny32_kernel<DT, 2>), grid, block, 0, st, g);
+        return status_of(hipGetLastError());
+    }
     if (p.cfg == 7) {
         const bool ok = p.bm == 16 ? launch_skinny<DT, 1>(g, p, st)
                         : p.bm == 32 ? launch_skinny<DT, 2>(g, p, st)

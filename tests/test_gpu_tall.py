@@ -1,0 +1,43 @@
+"""The 32-row kernel of the skinny forward path (17-64 tokens, weights tall enough to fill the chip
+with its 160-row workgroups): ragged rows (a segment's last workgroup, its last row tile), both
+token groups partly full, an odd number of super-steps (the second k-part one short), bias and
+LoRA, against fp32 products of the dequantized weight and, with one-hot rows, against the weight
+bit for bit.  The planner takes it here: its workgroups need one round of the 256 CUs, the 16-row
+kernel's two."""
+
+import pytest
+import torch
+
+from tests.gpu_util import assert_rel, banner, random_weight
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,m", [([18950, 18933], 256, 64), ([40000], 384, 33),
+                                      ([18944, 18944], 640, 17), ([37770], 256, 32),
+                                      ([18944, 18944], 384, 47)])
+def test_tall_forward(cuda, dtype, rows, k, m):
+    from solution import kernels
+
+    banner("tall fwd", dtype, rows, k, m)
+    weights = [random_weight(n, k, seed=500 + i, dev=cuda) for i, n in enumerate(rows)]
+    w = kernels.dequant(weights, dtype)
+    n = sum(rows)
+    g = torch.Generator(device=cuda).manual_seed(5)
+    buf = torch.full((m, k + 8), float("nan"), dtype=dtype, device=cuda)
+    x = buf[:, :k]
+    x.copy_(torch.randn(m, k, generator=g, device=cuda))
+    bias = torch.randn(n, generator=g, device=cuda).to(dtype)
+    for r in (16, 20):
+        t = torch.randn(m, r, generator=g, device=cuda).to(dtype)
+        b = (torch.randn(rows[-1], r, generator=g, device=cuda) * 0.05).to(dtype)
+        ref = x.float() @ w.float().T + bias.float()
+        ref[:, n - rows[-1]:] += 0.5 * t.float() @ b.float().T
+        y = kernels.linear_fwd(x, weights, bias, [kernels.make_lora(len(rows) - 1, r, 0.5, t=t, b=b)])
+        assert_rel(y, ref, what=f"y rank {r}")
+    for c0 in range(0, k, m):
+        idx = (torch.arange(m, device=cuda) + c0) % k
+        hot = torch.zeros(m, k, dtype=dtype, device=cuda)
+        hot[torch.arange(m, device=cuda), idx] = 1
+        assert torch.equal(kernels.linear_fwd(hot, weights), w.T[idx]), c0
