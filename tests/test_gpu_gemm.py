@@ -367,6 +367,30 @@ def test_lora_xa_decode_sizes(cuda, dtype, m, k, r):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,r", [(1, 8, 16), (3, 4104, 16), (17, 2048, 5), (33, 6152, 8), (63, 8960, 16)])
+def test_lora_xa_decode_step_edges(cuda, dtype, m, k, r):
+    """t = x A^T at decode token counts where the reduction ends in the first or the second of the
+    steps loaded together, one past them, and where lanes past K load the row's start: an
+    infinity there reaches its own token once and no other, and the next buffer's NaN nothing."""
+    from solution import kernels
+
+    banner("lora xa steps", dtype, m, k, r)
+    buf = torch.full((m + 8, k + 8), float("nan"), dtype=dtype, device=cuda)
+    x = buf[:m, :k]
+    x.copy_(_x(m, k, 57, cuda, dtype))
+    g = torch.Generator().manual_seed(58)
+    a = ((torch.rand(r, k, generator=g) + 0.5) / k ** 0.5).to(dtype).to(cuda)
+    t = torch.empty(m, r, dtype=dtype, device=cuda)
+    kernels.lora_xa_multi([kernels.lora_job(x, a, t)], m, r, dtype, x)
+    assert_rel(t, x.float().cpu() @ a.float().cpu().t(), what="xa")
+    x[0, 0] = float("inf")
+    t_inf = torch.empty_like(t)
+    kernels.lora_xa_multi([kernels.lora_job(x, a, t_inf)], m, r, dtype, x)
+    assert bool((t_inf[0] == float("inf")).all())
+    assert torch.equal(t_inf[1:], t[1:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("m,k,r", [(1, 1536, 16), (37, 3584, 16), (300, 1536, 64), (19, 200, 5)])
 def test_lora_ax(cuda, dtype, m, k, r):
     """d(xd) = scale * da A ([M, K]) for two jobs of different widths in one launch, against an
