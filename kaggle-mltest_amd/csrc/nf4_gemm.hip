@@ -3399,7 +3399,7 @@ int64_t dx_tail_col0(const Plan &p, int64_t m) {
 // From a thousand tokens or so on, dequantizing every weight tile again for each 256 tokens costs
 // more than writing the 16-bit weight to a workspace once (2.5 bytes per element at ~6.6 TB/s)
 // and multiplying it with a kernel free of dequantization (nf4_dense.hip).  Measured at M = 8192
-// (7B, bf16): gate|up forward 2109 -> 1799 us, its input gradient 2190 -> 1835, down 1123 -> 902;
+// (7B, bf16): gate|up forward 2047 -> 1677 us, its input gradient 1976 -> 1724, down 1123 -> 864;
 // at M = 512 the same products are 156 fused against 195.
 
 struct DenseRoute {
