@@ -197,7 +197,9 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
 
     // LoRA terms (of a split tile: split 0), 16 ranks at a time: the threads of waves 0-3 bring a
     // row p of the left operand each (dX: A's ranks are rows K apart, so the wave's loads of one
-    // rank coalesce), those of waves 4-7 a row m of the right one, 32 bytes per LDS row
+    // rank coalesce), those of waves 4-7 a row m of the right one, 32 bytes per LDS row.
+    // Rows p outside the slab take nothing, not even 0 * t, which is NaN where a token's t is not
+    // finite: a word per row masks the products (selects on the row index spill)
     for (int s = 0; s < (split > 0 ? 0 : a.nslab); ++s) {
         const DenseSlab &sl = a.slab[s];
         if (sl.p_hi <= p0 || sl.p_lo >= p0 + 128 * HP) continue;
@@ -214,6 +216,7 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
                 u32x4_t *dst = reinterpret_cast<u32x4_t *>(lds + (left ? 0 : 256 * 32) + r * 32);
                 dst[0] = slab8(src, step, in ? lim : 0, vec);
                 dst[1] = slab8(src + 8 * step, step, in ? lim - 8 : 0, vec);
+                if (left) *reinterpret_cast<uint32_t *>(lds + 512 * 32 + r * 4) = in ? ~0u : 0u;
             }
             __syncthreads();
 #pragma unroll
@@ -222,11 +225,19 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
                 for (int i = 0; i < 2; ++i) {
                     const u32x4_t fl = *reinterpret_cast<const u32x4_t *>(
                         lds + (h * 128 + wp * 64 + i * 32 + r32) * 32 + kh * 16);
+                    u32x4_t mask[4];
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; ++r4)
+                        mask[r4] = *reinterpret_cast<const u32x4_t *>(
+                            lds + 512 * 32 + (h * 128 + wp * 64 + i * 32 + r4 * 8 + kh * 4) * 4);
 #pragma unroll
                     for (int g = 0; g < HM; ++g) {
                         const u32x4_t ft = *reinterpret_cast<const u32x4_t *>(
                             lds + 256 * 32 + (g * 128 + wm * 32 + r32) * 32 + kh * 16);
-                        acc[h][g][i] += sl.scale * mfma32d<DT>(fl, ft, (float16_t){});
+                        const float16_t v = sl.scale * mfma32d<DT>(fl, ft, (float16_t){});
+#pragma unroll
+                        for (int e = 0; e < 16; ++e)
+                            acc[h][g][i][e] += __uint_as_float(__float_as_uint(v[e]) & mask[e / 4][e % 4]);
                     }
                 }
             __syncthreads();

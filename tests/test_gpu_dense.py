@@ -105,3 +105,33 @@ def test_dense_input_gradient(cuda, dtype, rows, k, m, splits):
     base = dx.clone()
     assert_rel(kernels.linear_dx(dy, weights, lora, out=base, accumulate=True),
                ref + dx.float(), what="accumulated dx")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,m,splits", FWD[:3])
+def test_dense_forward_keeps_non_finite_lora_to_its_segment(cuda, dtype, rows, k, m, splits):
+    """Slabs that start or end inside a tile, one token's t infinite and one's NaN: what lies
+    outside the slab's columns, and every other token, is as with a finite t, bit for bit."""
+    from solution import kernels
+
+    banner("dense fwd non-finite", dtype, rows, k, m, splits)
+    rows = rows if len(rows) > 1 else [72, rows[0] - 72]
+    weights, _ = _setup(rows, k, m, splits, dtype, cuda, False)
+    g = torch.Generator(device=cuda).manual_seed(6)
+    x = torch.randn(m, k, generator=g, device=cuda).to(dtype)
+    r, starts = 12, [0, rows[0]]
+    for seg in (0, 1):
+        t, b = _lora(m, r, k, rows[seg], dtype, cuda, 7 + seg)
+        b = b.abs() + 0.01  # (an infinity stays one)
+        bad = t.clone()
+        bad[5, 3], bad[m - 1] = float("inf"), float("nan")
+        y, y_bad = (kernels.linear_fwd(x, weights, None, [kernels.make_lora(seg, r, 0.5, t=v, b=b)])
+                    for v in (t, bad))
+        inside = torch.zeros(sum(rows), dtype=torch.bool, device=cuda)
+        inside[starts[seg]:starts[seg] + rows[seg]] = True
+        assert torch.equal(y_bad[:, ~inside], y[:, ~inside])
+        assert bool((y_bad[5, inside] == float("inf")).all())
+        assert bool(y_bad[m - 1, inside].isnan().all())
+        rest = torch.ones(m, dtype=torch.bool, device=cuda)
+        rest[5] = rest[m - 1] = False
+        assert torch.equal(y_bad[rest], y[rest])
