@@ -205,6 +205,24 @@ int nf4_linear_dx_tiled(const void *dy, int64_t m, int64_t lddy,
                         void *workspace, size_t workspace_bytes, void *stream,
                         int tile, int splits);
 
+/* The path that a call with the tiling chosen by the library takes: host code, nothing is
+ * launched and no pointer of `ws` is read through.  op NF4_OP_FWD (xa_rank: the largest rank of
+ * the adapters given with `a`, 0 for none) or NF4_OP_DX; outputs, LoRA tensors and the workspace
+ * (as large as its *_workspace call says) taken as aligned, nothing accumulated.  Returns
+ * NF4_PATH_*, or -1 for weights that the call refuses and empty products; *scratch, if given, the
+ * bytes of workspace that the call uses, never more than *_workspace returns.  For tests and
+ * profiles; which sizes take which path is no part of the interface. */
+#define NF4_OP_FWD 0
+#define NF4_OP_DX 1
+#define NF4_PATH_TILED 0     /* fused dequant-GEMM on 256x256 or 128x128 tiles */
+#define NF4_PATH_SMALL 1     /* small-M kernel */
+#define NF4_PATH_DECODE 2
+#define NF4_PATH_ROWS 3      /* row streaming */
+#define NF4_PATH_SKINNY 4    /* 16-row skinny kernel */
+#define NF4_PATH_SKINNY32 5  /* 32-row skinny kernel */
+#define NF4_PATH_DENSE 6     /* weight dequantized into the workspace, then a 16-bit GEMM */
+int nf4_linear_path(int64_t m, const nf4_weight *ws, int nw, int op, int xa_rank, size_t *scratch);
+
 /* ---------------------------------------------------------------------- LoRA side GEMMs */
 
 /* t[M, rank] = xd[M, K] @ A[rank, K]^T  (LoRA down-projection; layer.py:875, 877). */

@@ -3136,8 +3136,8 @@ constexpr double kFxCost = 2.0;
 
 // The skinny plan for the call: when it has LoRA down-projections to compute (xa_rank > 0: rank
 // of the largest), the best plan plus their own launch against the best plan that computes
-// them itself.  Either has no workspace when the plan without them has none, so the workspace
-// query, which does not see the adapters, stays valid.
+// them itself (which needs no workspace: one split).  So the call needs no more workspace than
+// the plan without adapters, which is what the workspace query sees.
 Plan choose_skinny(int64_t m, const nf4_weight *ws, int nw, int xa_rank, double *cost) {
     double t = 0;
     Plan p = plan_skinny(m, ws, nw, &t);
@@ -3178,8 +3178,10 @@ Plan plan_skinny32(int64_t m, const nf4_weight *ws, int nw, double *cost) {
 }
 
 // rows_allowed: the row-streaming path's operand alignment holds (LoRA T and B read as dwords).
-// xa_rank: the call's LoRA adapters ask for their down-projections (rank of the largest), which
-// only moves the choice between the skinny and decode paths (neither needs a workspace).
+// xa_rank: the call's LoRA adapters ask for their down-projections (rank of the largest).  It
+// moves the choice between the kernels of up to 64 tokens, but never to a plan that needs more
+// workspace than the plan without adapters: of those kernels only the 16-row skinny one splits,
+// and it is taken with splits only where it is taken without adapters too.
 Plan plan_fwd(int64_t m, const nf4_weight *ws, int nw, int tile = -1, int splits = 1,
               bool rows_allowed = true, int xa_rank = 0) {
     if (tile < 0 && rows_allowed && rows_ok(m, ws, nw)) return plan_rows(m, ws, nw);
@@ -3188,7 +3190,12 @@ Plan plan_fwd(int64_t m, const nf4_weight *ws, int nw, int tile = -1, int splits
         const Plan p = choose_skinny(m, ws, nw, xa_rank, &t);
         if (m <= 16) return p;
         const Plan p32 = plan_skinny32(m, ws, nw, &t32);
-        return t32 + (xa_rank > 0 ? xa_launch_cost(ws[0].cols) : 0.0) < 0.95 * t ? p32 : p;
+        // The adapters' own launch counts where the 16-row plan does without it.  Where both
+        // need it, p is the plan without adapters, and so is its time, to the last bit: with the
+        // launch on both sides of the 0.95 the choice would hang on the adapters.
+        if (xa_rank > 0 && skinny_fx_ok(p, xa_rank)) t32 += xa_launch_cost(ws[0].cols);
+        else plan_skinny(m, ws, nw, &t);
+        return t32 < 0.95 * t ? p32 : p;
     }
     if (tile < 0 && m <= kDecodeMaxM && ws[0].cols % DK == 0) return plan_decode(ws, nw);
     if (tile < 0 && m <= kGemvMaxM) return plan_gemv(m, ws, nw);
@@ -3394,6 +3401,18 @@ int64_t dx_tail_col0(const Plan &p, int64_t m) {
     return (p.tail_start / mt) * p.bp;
 }
 
+// Bytes of a split plan's fp32 partials: splits x M x the columns of its split tail.
+size_t fwd_partials(const Plan &p, int64_t m, const nf4_weight *ws, int nw) {
+    if (p.splits <= 1) return 0;
+    int64_t n = 0;
+    for (int i = 0; i < nw; ++i) n += ws[i].rows;
+    return static_cast<size_t>(p.splits) * m * (n - fwd_tail_col0(p, m, ws, nw)) * sizeof(float);
+}
+
+size_t dx_partials(const Plan &p, int64_t m, int64_t K) {
+    return p.splits > 1 ? static_cast<size_t>(p.splits) * m * (K - dx_tail_col0(p, m)) * sizeof(float) : 0;
+}
+
 // ------------------------------------------------- dequantized once, multiplied densely
 //
 // From a thousand tokens or so on, dequantizing every weight tile again for each 256 tokens costs
@@ -3504,14 +3523,9 @@ extern "C" size_t nf4_linear_fwd_workspace(int64_t m, const nf4_weight *ws, int 
     if (!ws || nw < 1 || nw > kMaxSeg || m <= 0) return 0;
     const Plan p = plan_fwd(m, ws, nw);
     const DenseRoute dense = dense_route_fwd(m, ws, nw, p);
-    size_t need = dense.use ? dense.bytes : 0;
-    if (p.splits > 1) {  // (also where the dense route is taken: a call that it does not fit)
-        int64_t n = 0;
-        for (int i = 0; i < nw; ++i) n += ws[i].rows;
-        const size_t fused = static_cast<size_t>(p.splits) * m * (n - fwd_tail_col0(p, m, ws, nw)) * sizeof(float);
-        if (fused > need) need = fused;
-    }
-    return need;
+    // (the partials also where the dense route is taken: a call that it does not fit)
+    const size_t fused = fwd_partials(p, m, ws, nw);
+    return dense.use && dense.bytes > fused ? dense.bytes : fused;
 }
 
 extern "C" size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int nw, int dtype) {
@@ -3519,9 +3533,33 @@ extern "C" size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int n
     if (!ws || nw < 1 || nw > kMaxSeg || m <= 0) return 0;
     const Plan p = plan_dx(m, ws, nw);
     const DenseRoute dense = dense_route_dx(m, ws, nw, p);
-    const size_t fused =
-        p.splits > 1 ? static_cast<size_t>(p.splits) * m * (ws[0].cols - dx_tail_col0(p, m)) * sizeof(float) : 0;
+    const size_t fused = dx_partials(p, m, ws[0].cols);
     return dense.use && dense.bytes > fused ? dense.bytes : fused;
+}
+
+extern "C" int nf4_linear_path(int64_t m, const nf4_weight *ws, int nw, int op, int xa_rank, size_t *scratch) {
+    GemmArgs g;
+    alignas(16) static const uint16_t row[8] = {};  // (an aligned address, never read)
+    if (m <= 0 || xa_rank < 0 || xa_rank > 64 || (op != NF4_OP_FWD && op != NF4_OP_DX) ||
+        fill_common(g, row, m, ws && nw > 0 ? (ws[0].cols + 7) / 8 * 8 : 0, ws, nw) != NF4_OK)
+        return -1;
+    int64_t n = 0;
+    for (int i = 0; i < nw; ++i) n += ws[i].rows;
+    if (n == 0 || g.K == 0) return -1;
+    size_t unused;
+    size_t &need = scratch ? *scratch : unused;
+    if (op == NF4_OP_DX) {
+        const Plan p = plan_dx(m, ws, nw);
+        const DenseRoute dense = dense_route_dx(m, ws, nw, p);
+        need = dense.use ? dense.bytes : dx_partials(p, m, g.K);
+        return dense.use ? NF4_PATH_DENSE : NF4_PATH_TILED;
+    }
+    const Plan p = plan_fwd(m, ws, nw, NF4_TILE_AUTO, 1, true, xa_rank);
+    const DenseRoute dense = dense_route_fwd(m, ws, nw, p);
+    need = dense.use ? dense.bytes : p.cfg == 6 ? 0 : fwd_partials(p, m, ws, nw);  // (row streaming adds in LDS)
+    if (dense.use) return NF4_PATH_DENSE;
+    return p.cfg == 2 ? NF4_PATH_SMALL : p.cfg == 4 ? NF4_PATH_DECODE : p.cfg == 6 ? NF4_PATH_ROWS
+         : p.cfg == 7 ? NF4_PATH_SKINNY : p.cfg == 8 ? NF4_PATH_SKINNY32 : NF4_PATH_TILED;
 }
 
 extern "C" int nf4_linear_fwd_tiled(const void *x, int64_t m, int64_t ldx, const nf4_weight *ws,
@@ -3650,8 +3688,7 @@ extern "C" int nf4_linear_fwd_tiled(const void *x, int64_t m, int64_t ldx, const
     g.tail_col0 = p.splits > 1 ? fwd_tail_col0(p, m, ws, nw) : n_out;
     g.tail_cols = n_out - g.tail_col0;
     if (p.splits > 1) {
-        const size_t need = static_cast<size_t>(p.splits) * m * g.tail_cols * sizeof(float);
-        if (!workspace || workspace_bytes < need) return NF4_ERR_WORKSPACE;
+        if (!workspace || workspace_bytes < fwd_partials(p, m, ws, nw)) return NF4_ERR_WORKSPACE;
         g.partial = static_cast<float *>(workspace);
     }
     if (p.head_ptiles > 0) {
@@ -3740,8 +3777,7 @@ int linear_dx_impl(const void *dy, int64_t m, int64_t lddy, const nf4_weight *ws
     g.tail_col0 = p.splits > 1 ? dx_tail_col0(p, m) : g.K;
     g.tail_cols = g.K - g.tail_col0;
     if (p.splits > 1) {
-        const size_t need = static_cast<size_t>(p.splits) * m * g.tail_cols * sizeof(float);
-        if (!workspace || workspace_bytes < need) return NF4_ERR_WORKSPACE;
+        if (!workspace || workspace_bytes < dx_partials(p, m, g.K)) return NF4_ERR_WORKSPACE;
         g.partial = static_cast<float *>(workspace);
     }
     if (p.head_ptiles > 0) {

@@ -82,6 +82,8 @@ _SIGNATURES = {
     "nf4_linear_dx_tiled": (c_int, [c_void_p, c_int64, c_int64, ctypes.POINTER(NF4Weight), c_int,
                                     ctypes.POINTER(NF4Lora), c_int, c_void_p, c_int64, c_int,
                                     c_int, c_void_p, c_size_t, c_void_p, c_int, c_int]),
+    "nf4_linear_path": (c_int, [c_int64, ctypes.POINTER(NF4Weight), c_int, c_int, c_int,
+                                ctypes.POINTER(c_size_t)]),
     "nf4_linear_swiglu_fwd": (c_int, [c_void_p, c_int64, c_int64, ctypes.POINTER(NF4Weight),
                                       c_void_p, c_int64, c_int, c_void_p]),
     "nf4_linear_swiglu_bwd": (c_int, [c_void_p, c_int64, c_int64, ctypes.POINTER(NF4Weight),

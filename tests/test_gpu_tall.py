@@ -41,3 +41,27 @@ def test_tall_forward(cuda, dtype, rows, k, m):
         hot = torch.zeros(m, k, dtype=dtype, device=cuda)
         hot[torch.arange(m, device=cuda), idx] = 1
         assert torch.equal(kernels.linear_fwd(hot, weights), w.T[idx]), c0
+
+
+def test_tall_forward_with_down_projection_where_the_kernels_cross(cuda):
+    """A size at which the 32-row kernel and a split 16-row one are nearly as fast: the adapter's
+    own launch for t = x A^T does not move the call to the plan whose partials the workspace
+    query, which does not see adapters, left out."""
+    from solution import kernels
+    from solution.quant_state import NF4_CODE, QuantState
+
+    rows, k, m, r, dtype = 33792, 8192, 17, 32, torch.bfloat16
+    banner("tall fwd with a", rows, k, m, r)
+    g = torch.Generator(device=cuda).manual_seed(8)
+    packed = torch.randint(0, 256, (rows * k // 2,), generator=g, device=cuda, dtype=torch.uint8)
+    absmax = torch.rand(rows * k // 64, generator=g, device=cuda) * 0.04 + 0.01
+    qs = QuantState(absmax=absmax, shape=torch.Size((rows, k)), dtype=dtype, blocksize=64,
+                    code=torch.tensor(NF4_CODE, device=cuda), quant_type="nf4")
+    x = torch.randn(m, k, generator=g, device=cuda).to(dtype)
+    a = (torch.randn(r, k, generator=g, device=cuda) / k ** 0.5).to(dtype)
+    b = (torch.randn(rows, r, generator=g, device=cuda) * 0.05).to(dtype)
+    t = torch.empty(m, r, dtype=dtype, device=cuda)
+    y = kernels.linear_fwd(x, [(packed, qs)], None, [kernels.make_lora(0, r, 0.5, t=t, b=b, a=a)])
+    w = kernels.dequant([(packed, qs)], dtype)
+    assert_rel(t, (x.float() @ a.float().T), what="t")
+    assert_rel(y, x.float() @ w.float().T + 0.5 * t.float() @ b.float().T, what="y")

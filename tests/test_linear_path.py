@@ -1,0 +1,50 @@
+"""The choice of a kernel path and the workspace queries, on the host (no GPU needed): whatever
+path a call takes, with or without adapters that ask for their down-projection, the workspace
+that the query returned for its sizes is enough."""
+
+import ctypes
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from solution import _lib
+
+    return _lib.load()
+
+
+def _weights(shapes, blocksize=64):
+    """Descriptors of stacked [rows, cols] weights; the addresses are aligned, and not read."""
+    from solution._lib import NF4Weight
+
+    at = 1 << 12
+    return (NF4Weight * len(shapes))(*[
+        NF4Weight(packed=at, absmax=at, absmax2=at, code2=at, code=at, nested=1, rows=r, cols=c,
+                  blocksize=blocksize, blocksize2=256) for r, c in shapes])
+
+
+FWD, DX = 0, 1
+TILED, SMALL, DECODE, ROWS, SKINNY, SKINNY32, DENSE = range(7)
+
+
+def path(lib, shapes, m, op=FWD, rank=0):
+    """(path, bytes of scratch it uses, bytes the query returns)."""
+    ws = _weights(shapes)
+    scratch = ctypes.c_size_t(0)
+    p = lib.nf4_linear_path(m, ws, len(shapes), op, rank, ctypes.byref(scratch))
+    query = lib.nf4_linear_dx_workspace if op == DX else lib.nf4_linear_fwd_workspace
+    return p, scratch.value, query(m, ws, len(shapes), 0)
+
+
+@pytest.mark.parametrize("rank", [0, 5, 16, 17, 64])
+def test_the_workspace_query_covers_every_forward_path(lib, rank):
+    seen = set()
+    for rows in [256, 1536, 4608, 16384, 29952, 33792, 35072, 37888, 41024, 52032, 65664, 81920]:
+        for k in [256, 1536, 3584, 4992, 8192, 8960, 16384, 18944]:
+            for m in [1, 2, 3, 8, 9, 16, 17, 24, 32, 33, 48, 64, 65, 512, 1300]:
+                for shapes in ([(rows, k)], [(rows // 2, k)] * 2):
+                    p, used, query = path(lib, shapes, m, rank=rank)
+                    assert p >= 0 and used <= query, (shapes, m, rank, p, used, query)
+                    seen.add(p)
+    assert seen == {TILED, DECODE, ROWS, SKINNY, SKINNY32, DENSE}
