@@ -139,7 +139,7 @@ int nf4_dequant_table(const void *dev_table, int nw, int64_t blocks, int out_dty
  *           addmm / mm projection GEMMs of FusedDecoderLayer.forward with the LoRA terms
  *           (layer.py:871-878, 893, 914, 929); RecomputedMLP's forward GEMMs (mlp.py:47-54).
  * workspace may be NULL when nf4_linear_fwd_workspace() returns 0 for the same arguments.  From
- * 512 tokens on, where it is faster, the call dequantizes the stacked weight into the
+ * 512 tokens on (below 2^23), where it is faster, the call dequantizes the stacked weight into the
  * workspace (2 bytes per element, rows padded to 128) and multiplies it there: 16-byte aligned
  * outputs with a row stride of a multiple of 8 and a 256-byte aligned workspace take that route,
  * others the fused one, for which the same workspace suffices. */

@@ -3442,10 +3442,11 @@ double fused_time(const Plan &p, int64_t small_tiles, int extra_segs) {
 // Taken where it is 4 % faster by the two models (10 % with a split reduction, whose partials
 // come on top of the weight in the workspace): of 308 measured (projection, direction, M, dtype)
 // points no fused one faster by more than 1 % is given up.  Below 512 tokens the
-// dequantization alone costs what the fused kernels need.
+// dequantization alone costs what the fused kernels need; from 2^23 on the dense kernel's 32-bit
+// tile arithmetic (band_tile: token tiles squared / 5) would come near its end.
 DenseRoute dense_route(int64_t P, int64_t m, int64_t R, double dequant_us, double fused_us) {
     DenseRoute r{};
-    if (m < 512 || (P + 127) * R >= (int64_t(1) << 30)) return r;
+    if (m < 512 || m >= (int64_t(1) << 23) || (P + 127) * R >= (int64_t(1) << 30)) return r;
     r.plan = dense_plan(P, m, R);
     r.use = r.plan.cost + dequant_us < (r.plan.splits > 1 ? 0.90 : 0.96) * fused_us;
     r.weight_bytes = static_cast<size_t>((P + 127) / 128) * 256 * R;  // strips (nf4_dense.h)

@@ -48,3 +48,22 @@ def test_the_workspace_query_covers_every_forward_path(lib, rank):
                     assert p >= 0 and used <= query, (shapes, m, rank, p, used, query)
                     seen.add(p)
     assert seen == {TILED, DECODE, ROWS, SKINNY, SKINNY32, DENSE}
+
+
+@pytest.mark.parametrize("op", [FWD, DX])
+def test_dense_tiles_are_counted_in_32_bits(lib, op):
+    """The dense kernel finds its tile in 32-bit arithmetic (band_tile in nf4_dense.hip: products of
+    up to tile rows x bands of about five): no call whose products could wrap takes it."""
+    dense = 0
+    for n in (12, 16, 18, 20, 22, 23, 24, 25, 26, 28, 30):
+        for m in ((1 << n) - 1, 1 << n, 38_000_000):
+            for shapes in ([(896, 896), (128, 896), (128, 896)], [(1536, 1536)], [(4864, 896)] * 2,
+                           [(896, 4864)], [(3584, 3584), (512, 3584), (512, 3584)]):
+                if path(lib, shapes, m, op)[0] != DENSE:
+                    continue
+                dense += 1
+                for tile in (128, 256):
+                    mt = -(-m // tile)
+                    bands = 1 if mt < 8 else (mt + 2) // 5
+                    assert (mt + 1) * bands < 1 << 32, (shapes, m)
+    assert dense > 20
