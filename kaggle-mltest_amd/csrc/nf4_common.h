@@ -371,6 +371,18 @@ __device__ __forceinline__ uint32_t bload2(rsrc_t r, int off) {
 __device__ __forceinline__ uint32_t bload1(rsrc_t r, int off) {
     return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, 0);
 }
+// LDS DMA: lane l's 16 bytes at `off` + `soff` of the resource to LDS address `lds` + 16 l (lds, soff
+// uniform).  As inline assembly: the compiler does not count these loads, so none of its own waits
+// also waits for them; each user waits for them itself.  M0 needs one wait state between a
+// scalar write and the DMA that reads it, which the compiler inserts after its own writes only.
+// M0 is declared clobbered (hipcc notes that it is a reserved register): nothing else in the
+// kernels that use this uses M0, so no value of the compiler's lives in it across the statement.
+__device__ __forceinline__ void lds_dma16(uint32_t lds, int off, rsrc_t r, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(off), "s"(r), "s"(soff)
+                 : "memory", "m0");
+}
 
 static inline int status_of(hipError_t e) { return e == hipSuccess ? NF4_OK : NF4_ERR_LAUNCH; }
 

@@ -100,14 +100,8 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
     auto send = [&](const rsrc_t &rs, const int (&o)[2], int half, int u) {
         const int kb = (u < u1 ? u : u1 - 1) * (half < HP ? HALF : 128);  // past the end: a reload nobody reads
         const uint32_t base = __builtin_amdgcn_readfirstlane(lds0 + ((u - u0) % NB) * BUF + half * HALF);
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     :
-                     : "s"(base), "v"(o[0]), "s"(rs), "s"(kb)
-                     : "memory", "m0");
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     :
-                     : "s"(base + 1024), "v"(o[1]), "s"(rs), "s"(kb)
-                     : "memory", "m0");
+        lds_dma16(base, o[0], rs, kb);
+        lds_dma16(base + 1024, o[1], rs, kb);
     };
     auto w0 = [&](int u) { send(rw0, wo, 0, u); };
     auto w1 = [&](int u) { send(rw1, wo, 1, u); };

@@ -1047,22 +1047,14 @@ __device__ __forceinline__ void fwd_body(const GemmArgs &a, const TileMap &tm, u
     const uint32_t lds_a =  // this wave's activation rows in the group's LDS stage 0
         static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds)) +
         (g * NS * (BP + BM) + BP + wave * CHA * 8) * ROWB;
-    // The DMA as inline assembly: the compiler does not count these loads, so none of its own
-    // waits (for the weight registers) also waits for them; wait_dma() waits for them instead.
-    // M0 is declared clobbered (hipcc notes that it is a reserved register): nothing else in
-    // these kernels uses M0, so no value of the compiler's lives in it across the statement.
+    // (the compiler's own waits, for the weight registers, do not wait for the DMA: wait_dma() does)
     auto dma_a = [&](int b, int64_t v) {  // activations of step v into LDS stage b
         const int64_t st = s0 + g + KG * v;
         const rsrc_t rs = KG > 1 && st >= s1 ? ar0 : ar;
         const int kb = static_cast<int>(st) * (BR * 2);
         const uint32_t base = __builtin_amdgcn_readfirstlane(lds_a + b * (BP + BM) * ROWB);
 #pragma unroll
-        for (int j = 0; j < CHA; ++j) {
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         :
-                         : "s"(base + j * 8 * ROWB), "v"(adoff[j]), "s"(rs), "s"(kb)
-                         : "memory", "m0");
-        }
+        for (int j = 0; j < CHA; ++j) lds_dma16(base + j * 8 * ROWB, adoff[j], rs, kb);
     };
     // Every DMA is followed by exactly the 3 global loads of one weight register stage (packed
     // bytes, absmax code, absmax scale) and by nothing else before this wait, and loads complete
@@ -1249,12 +1241,7 @@ __device__ __forceinline__ void fwd_body_rw(const GemmArgs &a, const TileMap &tm
         const int kb = static_cast<int>(s0 + u) * (BR * 2);
         const uint32_t base = __builtin_amdgcn_readfirstlane(lds_a + b * STG);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         :
-                         : "s"(base + j * 8 * ROWB), "v"(adoff[j]), "s"(ar), "s"(kb)
-                         : "memory", "m0");
-        }
+        for (int j = 0; j < 4; ++j) lds_dma16(base + j * 8 * ROWB, adoff[j], ar, kb);
     };
     // Every DMA is followed by exactly one register stage's 3 loads before this wait.
     auto wait_dma = [] { asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); };
@@ -2572,12 +2559,7 @@ __device__ __forceinline__ void dx_body(const GemmArgs &a, const TileMap &tm, ui
             const int kb = static_cast<int>((col_base + (st - first) * BR) * 2);
             const uint32_t base = __builtin_amdgcn_readfirstlane(lds_a + b * (BP + BM) * ROWB);
 #pragma unroll
-            for (int j = 0; j < CHA; ++j) {
-                asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                             :
-                             : "s"(base + j * 8 * ROWB), "v"(adoff[j]), "s"(rs), "s"(kb)
-                             : "memory", "m0");
-            }
+            for (int j = 0; j < CHA; ++j) lds_dma16(base + j * 8 * ROWB, adoff[j], rs, kb);
         };
         auto stage = [&](int b, int64_t v) { wt[b].load(wr, wa, (b0 + g + KG * v - first) * BR, K); };
         // After the DMA of step v into stage b has landed and the barrier: zero its columns past

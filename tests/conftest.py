@@ -24,10 +24,8 @@ def cuda():
     return torch.device("cuda:0")
 
 
-@pytest.fixture(scope="session")
-def gemm_asm(tmp_path_factory):
-    """nf4_gemm.hip compiled for gfx950 to assembly, once per session (hipcc cross-compiles
-    without a GPU): the text, read by the tests of register counts and wait placement."""
+def _assembly(name, tmp_path_factory):
+    """csrc/<name>.hip compiled for gfx950 to assembly text (hipcc cross-compiles without a GPU)."""
     import subprocess
 
     import build
@@ -36,12 +34,25 @@ def gemm_asm(tmp_path_factory):
         hipcc = build.hipcc()
     except RuntimeError:
         pytest.skip("hipcc not available")
-    out = tmp_path_factory.mktemp("asm") / "nf4_gemm.s"
-    cmd = [hipcc, *build.FLAGS, "--offload-device-only", "-S", str(PKG / "csrc" / "nf4_gemm.hip"),
+    out = tmp_path_factory.mktemp("asm") / f"{name}.s"
+    cmd = [hipcc, *build.FLAGS, "--offload-device-only", "-S", str(PKG / "csrc" / f"{name}.hip"),
            "-o", str(out)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
     return out.read_text()
+
+
+@pytest.fixture(scope="session")
+def gemm_asm(tmp_path_factory):
+    """nf4_gemm.hip's assembly, once per session: read by the tests of register counts and wait
+    placement."""
+    return _assembly("nf4_gemm", tmp_path_factory)
+
+
+@pytest.fixture(scope="session")
+def dense_asm(tmp_path_factory):
+    """nf4_dense.hip's assembly, once per session."""
+    return _assembly("nf4_dense", tmp_path_factory)
 
 
 def pytest_collection_modifyitems(config, items):

@@ -199,6 +199,20 @@ def test_no_register_of_a_load_in_flight_is_touched(kernels):
         assert not hz, f"{name}: {hz[:3]}"
 
 
+@pytest.mark.timeout(600)
+def test_m0_is_settled_before_the_dma_reads_it(gemm_asm, dense_asm):
+    """LDS DMA takes its LDS address from M0 and needs one wait state after a scalar write of it;
+    the compiler puts one after its own writes, an inline-assembly statement has to itself."""
+    checked = 0
+    for name, body in _kernels(gemm_asm) + _kernels(dense_asm):
+        lines = [t for t in _strip(body) if not t.endswith(":")]
+        for before, t in zip(lines, lines[1:]):
+            if _is_dma(t):
+                assert not re.match(r"s_\w+ m0\b", before), f"{name}: {before} / {t}"
+                checked += 1
+    assert checked > 200
+
+
 def test_replay_model_flags_a_register_used_before_its_wait():
     """The model itself: a load whose register is read before a wait covers it is flagged; the
     same read after vmcnt(0), or after a vmcnt(1) that leaves only a younger load in flight, is
