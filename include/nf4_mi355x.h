@@ -8,7 +8,8 @@
  * one entry point the library owns no device memory and keeps no state between calls, so it is
  * reentrant and thread-safe.  The exception is nf4_linear_dx_noalloc (for callers that cannot
  * allocate): its workspace is a 64 MiB device array that the library holds on every
- * GPU it runs on until the process ends, and calls of it that overlap on one GPU race.
+ * GPU it runs on until the process ends, and calls of it that use that array and overlap on one
+ * GPU race.
  *
  * Weight format (bitsandbytes 0.50.2 QuantState, as read by the reference at
  * /root/reference/solution/nf4.py:46-53,112-131):
@@ -167,11 +168,15 @@ size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int nw, int dtyp
  * forbid allocation).  No counterpart in the reference.  Its workspace is one static
  * device array of NF4_STATIC_SCRATCH_BYTES per GPU, set up when the library's code loads on a
  * device and held until the process ends; its address is looked up on the first call on each
- * device (make that first call outside graph capture).  The plan is nf4_linear_dx's where its
- * workspace fits the array, else the best fused tiling whose partials do, so every size
- * is accepted; the result equals nf4_linear_dx's bit for bit whenever its plan fits.  The
- * array keeps the last call's contents; calls that overlap on one GPU (other streams or
- * threads) share it and race.  The stream must belong to the current device. */
+ * device (make that first call outside graph capture).  The fused tiling is chosen among those
+ * whose partials fit the array (tilings with no split need none), so every size is accepted;
+ * where that tiling is split and nf4_linear_dx dequantizes the weight into its workspace, the
+ * call does so too if it fits.  The result equals nf4_linear_dx's bit for bit whenever what that
+ * call keeps in its workspace fits, except where it dequantizes there and the fused tiling is
+ * not split: these calls stay fused, use no scratch and may overlap (nf4_linear_path with
+ * NF4_OP_DX_NOALLOC tells: scratch 0).  The array keeps the last call's contents; calls that
+ * use it and overlap on one GPU (other streams or threads) race.  The stream must belong to the
+ * current device. */
 #define NF4_STATIC_SCRATCH_BYTES (64u << 20)
 int nf4_linear_dx_noalloc(const void *dy, int64_t m, int64_t lddy,
                           const nf4_weight *ws, int nw,
@@ -207,13 +212,15 @@ int nf4_linear_dx_tiled(const void *dy, int64_t m, int64_t lddy,
 
 /* The path that a call with the tiling chosen by the library takes: host code, nothing is
  * launched and no pointer of `ws` is read through.  op NF4_OP_FWD (xa_rank: the largest rank of
- * the adapters given with `a`, 0 for none) or NF4_OP_DX; outputs, LoRA tensors and the workspace
- * (as large as its *_workspace call says) taken as aligned, nothing accumulated.  Returns
- * NF4_PATH_*, or -1 for weights that the call refuses and empty products; *scratch, if given, the
- * bytes of workspace that the call uses, never more than *_workspace returns.  For tests and
- * profiles; which sizes take which path is no part of the interface. */
+ * the adapters given with `a`, 0 for none), NF4_OP_DX or NF4_OP_DX_NOALLOC; outputs, LoRA tensors
+ * and the workspace (as large as its *_workspace call says) taken as aligned, nothing
+ * accumulated.  Returns NF4_PATH_*, or -1 for weights that the call refuses and empty products;
+ * *scratch, if given, the bytes of workspace (of the static array) that the call uses, never more
+ * than *_workspace returns (NF4_STATIC_SCRATCH_BYTES).  For tests and profiles; which sizes take
+ * which path is no part of the interface. */
 #define NF4_OP_FWD 0
 #define NF4_OP_DX 1
+#define NF4_OP_DX_NOALLOC 2
 #define NF4_PATH_TILED 0     /* fused dequant-GEMM on 256x256 or 128x128 tiles */
 #define NF4_PATH_SMALL 1     /* small-M kernel */
 #define NF4_PATH_DECODE 2

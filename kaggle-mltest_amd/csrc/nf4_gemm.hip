@@ -3461,6 +3461,17 @@ DenseRoute dense_route_dx(int64_t m, const nf4_weight *ws, int nw, const Plan &p
                        fused_time(p, (K + 127) / 128 * ((m + 127) / 128), nw - 1));
 }
 
+// The same for a call whose fused plan is p.  nf4_linear_dx_noalloc (ws_cap >= 0: the bytes of its
+// array, to which p was restricted) takes it only where p would use the array too: calls whose
+// fused plan needs none stay independent of each other.
+DenseRoute dense_route_dx(int64_t m, const nf4_weight *ws, int nw, const Plan &p, int64_t ws_cap) {
+    if (ws_cap < 0) return dense_route_dx(m, ws, nw, p);
+    if (p.splits <= 1) return DenseRoute{};
+    DenseRoute r = dense_route_dx(m, ws, nw, plan_dx(m, ws, nw));
+    if (r.bytes > static_cast<size_t>(ws_cap)) r.use = false;
+    return r;
+}
+
 // The second launch of the dense route and, of a split plan, the reduction: g holds the call.
 int launch_dense(GemmArgs &g, const DenseRoute &r, int nw, bool dx, void *workspace, int dtype, hipStream_t s) {
     DenseArgs a = {};
@@ -3523,7 +3534,7 @@ extern "C" size_t nf4_linear_dx_workspace(int64_t m, const nf4_weight *ws, int n
 extern "C" int nf4_linear_path(int64_t m, const nf4_weight *ws, int nw, int op, int xa_rank, size_t *scratch) {
     GemmArgs g;
     alignas(16) static const uint16_t row[8] = {};  // (an aligned address, never read)
-    if (m <= 0 || xa_rank < 0 || xa_rank > 64 || (op != NF4_OP_FWD && op != NF4_OP_DX) ||
+    if (m <= 0 || xa_rank < 0 || xa_rank > 64 || op < NF4_OP_FWD || op > NF4_OP_DX_NOALLOC ||
         fill_common(g, row, m, ws && nw > 0 ? (ws[0].cols + 7) / 8 * 8 : 0, ws, nw) != NF4_OK)
         return -1;
     int64_t n = 0;
@@ -3531,9 +3542,10 @@ extern "C" int nf4_linear_path(int64_t m, const nf4_weight *ws, int nw, int op, 
     if (n == 0 || g.K == 0) return -1;
     size_t unused;
     size_t &need = scratch ? *scratch : unused;
-    if (op == NF4_OP_DX) {
-        const Plan p = plan_dx(m, ws, nw);
-        const DenseRoute dense = dense_route_dx(m, ws, nw, p);
+    if (op != NF4_OP_FWD) {
+        const int64_t ws_cap = op == NF4_OP_DX_NOALLOC ? int64_t(NF4_STATIC_SCRATCH_BYTES) : -1;
+        const Plan p = plan_dx(m, ws, nw, NF4_TILE_AUTO, 1, ws_cap);
+        const DenseRoute dense = dense_route_dx(m, ws, nw, p, ws_cap);
         need = dense.use ? dense.bytes : dx_partials(p, m, g.K);
         return dense.use ? NF4_PATH_DENSE : NF4_PATH_TILED;
     }
@@ -3738,16 +3750,16 @@ int linear_dx_impl(const void *dy, int64_t m, int64_t lddy, const nf4_weight *ws
     g.accumulate = accumulate != 0;
     g.vec_out = aligned(dx, 8) && lddx % 4 == 0;
     g.vec16_out = aligned(dx, 16) && lddx % 8 == 0;
+    const Plan p = plan_dx(m, ws, nw, tile, splits, ws_cap);
+    if (p.splits == 0) return NF4_ERR_ARG;
     if (tile < 0 && g.vec16_out && !accumulate && aligned(workspace, 256)) {
-        const DenseRoute dense = dense_route_dx(m, ws, nw, plan_dx(m, ws, nw));
+        const DenseRoute dense = dense_route_dx(m, ws, nw, p, ws_cap);
         if (dense.use && workspace && workspace_bytes >= dense.bytes) {
             hipStream_t s = static_cast<hipStream_t>(stream);
             st = dequant_strips(ws, nw, true, workspace, dtype, s);
             return st != NF4_OK ? st : launch_dense(g, dense, nw, true, workspace, dtype, s);
         }
     }
-    const Plan p = plan_dx(m, ws, nw, tile, splits, ws_cap);
-    if (p.splits == 0) return NF4_ERR_ARG;
     g.splits = p.splits;
     const int64_t bp = p.bp, bm = p.bm;
     g.map[0].m_tiles = (m + bm - 1) / bm;
@@ -3779,14 +3791,15 @@ int linear_dx_impl(const void *dy, int64_t m, int64_t lddy, const nf4_weight *ws
 
 // ------------------------------------------------- the allocation-free input gradient
 //
-// nf4_linear_dx_noalloc keeps its split-K partials in `scratch`, one array of
+// nf4_linear_dx_noalloc keeps its split-K partials, or the dense route's 16-bit weight and
+// partials, in `scratch`, one array of
 // NF4_STATIC_SCRATCH_BYTES per GPU, allocated when the library's code is loaded on a device
 // and held until the process ends.  In host code `scratch` names a host-side stand-in, not
 // device memory: its device address is looked up once per device (hipGetSymbolAddress, with
 // that device current, on the entry point's first call there) and only that address is used.
-// Every split tile writes all of its partials before the reduction reads them, so nothing in
-// the array needs clearing between calls.  Calls that overlap on one GPU (two streams, two
-// threads) share the array and race.
+// Every byte that a call reads there it has written before, so nothing in the array needs
+// clearing between calls.  Calls that use the array and overlap on one GPU (two streams, two
+// threads) race; those whose fused plan is not split do not touch it.
 
 static __device__ __align__(256) uint8_t scratch[NF4_STATIC_SCRATCH_BYTES];
 

@@ -24,7 +24,8 @@ def _weights(shapes, blocksize=64):
                   blocksize=blocksize, blocksize2=256) for r, c in shapes])
 
 
-FWD, DX = 0, 1
+FWD, DX, DX_NOALLOC = 0, 1, 2
+STATIC_SCRATCH = 64 << 20  # NF4_STATIC_SCRATCH_BYTES
 TILED, SMALL, DECODE, ROWS, SKINNY, SKINNY32, DENSE = range(7)
 
 
@@ -67,3 +68,26 @@ def test_dense_tiles_are_counted_in_32_bits(lib, op):
                     bands = 1 if mt < 8 else (mt + 2) // 5
                     assert (mt + 1) * bands < 1 << 32, (shapes, m)
     assert dense > 20
+
+
+def test_noalloc_shares_its_array_only_where_its_fused_plan_would(lib):
+    """nf4_linear_dx_noalloc dequantizes into its array only where its fused plan is split and
+    uses the array in any case: elsewhere a call has no scratch, so calls may overlap."""
+    shapes = ([(1536, 1536), (256, 1536), (256, 1536)], [(3584, 3584), (512, 3584), (512, 3584)],
+              [(3584, 3584)], [(1536, 8960)], [(3008, 1536), (64, 1536)], [(8960, 1536)] * 2,
+              [(18944, 3584)] * 2)
+    seen = set()
+    for s in shapes:
+        for m in (64, 300, 700, 1025, 1243, 1300, 2048, 2500, 3000, 4096, 6000, 8192):
+            p, used, query = path(lib, s, m, DX)
+            q, noalloc, _ = path(lib, s, m, DX_NOALLOC)
+            assert noalloc <= STATIC_SCRATCH, (s, m)
+            if q == DENSE:  # as nf4_linear_dx
+                assert p == DENSE and noalloc == used, (s, m)
+            elif p == DENSE:
+                assert noalloc == 0 or used > STATIC_SCRATCH, (s, m, noalloc)
+            elif query <= STATIC_SCRATCH:
+                assert noalloc == used, (s, m)
+            seen.add((p, q, noalloc > 0))
+    assert {(DENSE, TILED, False), (DENSE, DENSE, True), (TILED, TILED, False),
+            (TILED, TILED, True)} <= seen

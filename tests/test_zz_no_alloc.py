@@ -71,3 +71,80 @@ def test_noalloc_dx_matches_linear_dx(cuda):
     out3 = _noalloc(dy3, [gate, up], torch.empty_like(ref3))
     torch.cuda.synchronize()
     assert_rel(out3, ref3.float().cpu(), what="restricted plan")
+
+
+QKV_15B = [(1536, 1536), (256, 1536), (256, 1536)]
+QKV_7B = [(3584, 3584), (512, 3584), (512, 3584)]
+
+
+def _path(weights, m, op):
+    import ctypes
+
+    from solution import _lib, kernels
+
+    scratch = ctypes.c_size_t(0)
+    path = _lib.load().nf4_linear_path(m, kernels._descs(weights), len(weights), op, 0,
+                                       ctypes.byref(scratch))
+    return path, scratch.value
+
+
+def _problem(shapes, m, seed, dtype, dev):
+    weights = [random_weight(n, k, seed=seed + i, dev=dev) for i, (n, k) in enumerate(shapes)]
+    g = torch.Generator(device=dev).manual_seed(seed)
+    dy = (torch.randn(m, sum(n for n, _ in shapes), generator=g, device=dev) * 1e-3).to(dtype)
+    return weights, dy
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shapes,m", [(QKV_7B, 2500), ([(3584, 3584)], 3000)])
+def test_noalloc_on_the_dense_route_matches_linear_dx(cuda, dtype, shapes, m):
+    """The weight dequantized into the array (where the fused plan is split, and it fits): bit for
+    bit nf4_linear_dx's."""
+    from solution import kernels
+
+    banner("noalloc dense", dtype, shapes, m)
+    weights, dy = _problem(shapes, m, 900, dtype, cuda)
+    assert _path(weights, m, 1) == _path(weights, m, 2) and _path(weights, m, 2)[0] == 6
+    ref = kernels.linear_dx(dy, weights)
+    out = _noalloc(dy, weights, torch.full_like(ref, float("nan")))
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shapes,m", [(QKV_15B, 1025), (QKV_7B, 4096), ([(1536, 8960)], 4096)])
+def test_noalloc_without_scratch_is_the_fused_product(cuda, dtype, shapes, m):
+    """Sizes at which nf4_linear_dx dequantizes into its workspace but the fused plan needs none:
+    bit for bit nf4_linear_dx's result without a workspace."""
+    from solution import _lib, kernels
+
+    banner("noalloc unsplit", dtype, shapes, m)
+    weights, dy = _problem(shapes, m, 910, dtype, cuda)
+    assert _path(weights, m, 1)[0] == 6
+    ref = torch.empty(m, shapes[0][1], dtype=dtype, device=cuda)
+    _lib.check(_lib.load().nf4_linear_dx(
+        dy.data_ptr(), m, dy.stride(0), kernels._descs(weights), len(weights), None, 0,
+        ref.data_ptr(), ref.stride(0), 0, _lib.DTYPE_CODE[dtype], None, 0, _lib.stream_of(dy)),
+        "nf4_linear_dx")
+    out = _noalloc(dy, weights, torch.full_like(ref, float("nan")))
+    assert torch.equal(out, ref)
+
+
+def test_noalloc_calls_without_scratch_overlap(cuda):
+    """Two streams, two problems of a size that needs no scratch, several calls each in flight."""
+    m = 1025
+    problems = [_problem(QKV_15B, m, 920 + 10 * i, torch.float16, cuda) for i in range(2)]
+    assert _path(problems[0][0], m, 2)[1] == 0
+    banner("noalloc overlapping", QKV_15B, m)
+    outs = [[torch.full((m, 1536), float("nan"), dtype=torch.float16, device=cuda)
+             for _ in range(8)] for _ in problems]
+    refs = [_noalloc(dy, w, torch.empty_like(outs[0][0])) for w, dy in problems]
+    streams = [torch.cuda.Stream() for _ in problems]
+    torch.cuda.synchronize()
+    for i in range(8):
+        for (w, dy), out, st in zip(problems, outs, streams):
+            with torch.cuda.stream(st):
+                _noalloc(dy, w, out[i])
+    torch.cuda.synchronize()
+    for out, ref in zip(outs, refs):
+        for o in out:
+            assert torch.equal(o, ref)
