@@ -154,16 +154,18 @@ class ProjectionStack:
             raise ValueError(f"{m} tokens exceed the stack's max_tokens {self.max_tokens}")
         self.m = m
         lib, L0 = self.lib, self.per_layer[0]
-        need = {}
-        for g, _ in GROUPS:
-            need[g] = (lib.nf4_linear_fwd_workspace(m, L0[g], L0[g + "_n"], self.dt),
-                       lib.nf4_linear_dx_workspace(m, L0[g], L0[g + "_n"], self.dt))
-        need["wgrad"] = (lib.nf4_lora_wgrad_multi_workspace(L0["wg_jobs"], 4, m, self.rank), 0)
-        for key, (fb, db) in need.items():
+        # one workspace per direction: its launches run in order on one stream, and the largest
+        # product's dequantized weight is most of it (7B, 8192 tokens: 518 MiB in all, 951 with
+        # one per group)
+        need = {"fwd": max(lib.nf4_linear_fwd_workspace(m, L0[g], L0[g + "_n"], self.dt)
+                           for g, _ in GROUPS),
+                "dx": max(lib.nf4_linear_dx_workspace(m, L0[g], L0[g + "_n"], self.dt)
+                          for g, _ in GROUPS),
+                "wgrad": lib.nf4_lora_wgrad_multi_workspace(L0["wg_jobs"], 4, m, self.rank)}
+        for key, nbytes in need.items():
             have = self.ws.get(key)
-            if have is None or have[1] < fb or have[3] < db:
-                self.ws[key] = (torch.empty(max(fb, 1), dtype=torch.uint8, device=self.dev), fb,
-                                torch.empty(max(db, 1), dtype=torch.uint8, device=self.dev), db)
+            if have is None or have.numel() < nbytes:
+                self.ws[key] = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=self.dev)
         return m
 
     # ------------------------------------------------------------------------------ counts
@@ -206,21 +208,21 @@ class ProjectionStack:
         s = torch.cuda.current_stream(self.dev).cuda_stream
         P = lambda t: t.data_ptr()  # noqa: E731
         h, i, nq, r = self.shape.hidden, self.shape.inter, self.n_qkv, self.rank
-        ws = self.ws
+        ws, wb = P(self.ws["fwd"]), self.ws["fwd"].numel()
         for li in (range(len(self.per_layer)) if layers is None else layers):
             L = self.per_layer[li]
             self._timed(ev, "fwd_qkv", lambda: lib.nf4_linear_fwd(
                 P(self.x), m, h, L["qkv"], 3, P(L["bias"]), L["fwd_loras"], 2, P(self.y_qkv), nq,
-                dt, P(ws["qkv"][0]), ws["qkv"][1], s))
+                dt, ws, wb, s))
             self._timed(ev, "fwd_o", lambda: lib.nf4_linear_fwd(
                 P(self.attn), m, h, L["o"], 1, None, None, 0, P(self.y_o), h, dt,
-                P(ws["o"][0]), ws["o"][1], s))
+                ws, wb, s))
             self._timed(ev, "fwd_gu", lambda: lib.nf4_linear_fwd(
                 P(self.x2), m, h, L["gu"], 2, None, None, 0, P(self.y_gu), 2 * i, dt,
-                P(ws["gu"][0]), ws["gu"][1], s))
+                ws, wb, s))
             self._timed(ev, "fwd_down", lambda: lib.nf4_linear_fwd(
                 P(self.act), m, i, L["down"], 1, None, None, 0, P(self.y_d), h, dt,
-                P(ws["down"][0]), ws["down"][1], s))
+                ws, wb, s))
 
     def backward(self, ev=None, layers=None):
         """Queue the backward projections (input gradients and LoRA gradients), last layer
@@ -229,26 +231,26 @@ class ProjectionStack:
         s = torch.cuda.current_stream(self.dev).cuda_stream
         P = lambda t: t.data_ptr()  # noqa: E731
         h, i, nq, r = self.shape.hidden, self.shape.inter, self.n_qkv, self.rank
-        ws = self.ws
-        wg, wb = P(ws["wgrad"][0]), ws["wgrad"][1]
+        ws, wb = P(self.ws["dx"]), self.ws["dx"].numel()
+        wg, wgb = P(self.ws["wgrad"]), self.ws["wgrad"].numel()
         order = reversed(range(len(self.per_layer))) if layers is None else layers
         for li in order:
             L = self.per_layer[li]
             self._timed(ev, "dx_down", lambda: lib.nf4_linear_dx(
                 P(self.dy_d), m, h, L["down"], 1, None, 0, P(self.dx_d), i, 0, dt,
-                P(ws["down"][2]), ws["down"][3], s))
+                ws, wb, s))
             self._timed(ev, "dx_gu", lambda: lib.nf4_linear_dx(
                 P(self.dy_gu), m, 2 * i, L["gu"], 2, None, 0, P(self.dx_gu), h, 0, dt,
-                P(ws["gu"][2]), ws["gu"][3], s))
+                ws, wb, s))
             self._timed(ev, "dx_o", lambda: lib.nf4_linear_dx(
                 P(self.dy_o), m, h, L["o"], 1, None, 0, P(self.dx_o), h, 0, dt,
-                P(ws["o"][2]), ws["o"][3], s))
+                ws, wb, s))
             dq = P(self.dy_qkv)
             self._chk(lib.nf4_lora_da_multi(L["da_jobs"], 2, m, r, dt, s), "da")
-            self._chk(lib.nf4_lora_wgrad_multi(L["wg_jobs"], 4, m, r, dt, wg, wb, s), "wgrad")
+            self._chk(lib.nf4_lora_wgrad_multi(L["wg_jobs"], 4, m, r, dt, wg, wgb, s), "wgrad")
             self._timed(ev, "dx_qkv", lambda: lib.nf4_linear_dx(
                 dq, m, nq, L["qkv"], 3, L["dx_loras"], 2, P(self.dx_qkv), h, 0, dt,
-                P(ws["qkv"][2]), ws["qkv"][3], s))
+                ws, wb, s))
 
     def step(self, ev=None):
         self.forward(ev)

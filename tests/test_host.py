@@ -186,3 +186,21 @@ def test_apply_with_unloadable_library_keeps_bitsandbytes(monkeypatch, capsys, t
     assert after == before
     err = capsys.readouterr().err
     assert err.count("not applied: NF4LibraryError") == 3, err
+
+
+def test_stack_holds_one_workspace_per_direction():
+    """The launches of a direction run in order on one stream and share their workspace: the
+    stack holds the largest need of each direction, not one buffer per projection."""
+    from solution.stack import GROUPS, ProjectionStack, Qwen2Shape
+
+    st = ProjectionStack.synthetic(Qwen2Shape(hidden=1024, inter=2048, kv=128), 1, 48,
+                                   device="cpu")
+    L, fwd, dx = st.per_layer[0], [], []
+    for g, _ in GROUPS:
+        fwd.append(st.lib.nf4_linear_fwd_workspace(48, L[g], L[g + "_n"], st.dt))
+        dx.append(st.lib.nf4_linear_dx_workspace(48, L[g], L[g + "_n"], st.dt))
+    assert sum(n > 0 for n in dx) > 1
+    held = [t for v in st.ws.values() for t in (v if isinstance(v, tuple) else (v,))
+            if isinstance(t, torch.Tensor)]
+    wgrad = st.lib.nf4_lora_wgrad_multi_workspace(L["wg_jobs"], 4, 48, st.rank)
+    assert sum(t.numel() for t in held) <= max(fwd) + max(dx) + wgrad + len(held)
