@@ -163,13 +163,12 @@ def weight_desc(packed: torch.Tensor, quant_state) -> NF4Weight:
         refs = (dev, code, absmax, absmax2, code2, offset, bs2)
         qs._nf4_refs = refs
     _, code, absmax, absmax2, code2, offset, bs2 = refs
-    rows, cols = qs.shape
     return NF4Weight(
         packed.data_ptr(), absmax.data_ptr(),
         absmax2.data_ptr() if absmax2 is not None else None,
         code2.data_ptr() if code2 is not None else None,
-        code.data_ptr(), offset, 1 if qs.nested else 0, int(rows), int(cols),
-        int(qs.blocksize), bs2)
+        code.data_ptr(), offset, 1 if qs.nested else 0, int(qs.shape[0]),
+        int(qs.shape[1]), int(qs.blocksize), bs2)
 
 
 def weight_array(descs: list[NF4Weight]):

@@ -82,6 +82,16 @@ def test_weight_descriptor_fields():
     assert d.absmax == qs._nf4_refs[2].data_ptr()
 
 
+@pytest.mark.parametrize("shape", [(16, 256), (16, 256, 1), [16, 256], torch.Size((16, 256, 1))])
+def test_weight_descriptor_takes_the_first_two_dimensions(shape):
+    from solution.quant_state import quantize_4bit, weight_desc
+
+    packed, qs = quantize_4bit(torch.randn(16, 256))
+    qs.shape = shape
+    d = weight_desc(packed, qs)
+    assert (d.rows, d.cols) == (16, 256)
+
+
 def test_kernels_refuse_cpu_tensors_loudly():
     """No CPU fallback: the product path raises instead of computing on the host."""
     from solution.nf4 import NF4Linear, dequantize_nf4
