@@ -50,6 +50,23 @@ def random_weight(n, k, seed, dev, std=0.02, blocksize=64, nested=True):
     return packed.view(-1), qs
 
 
+# nf4_linear_path's operations and the paths asserted in tests (NF4_OP_*, NF4_PATH_* of the C header)
+OP_FWD, OP_DX, OP_DX_NOALLOC = 0, 1, 2
+PATH_SKINNY32, PATH_DENSE = 5, 6
+
+
+def linear_path(weights, m, op=OP_FWD, xa_rank=0):
+    """(NF4_PATH_*, bytes of scratch) of a product over `weights` with m tokens."""
+    import ctypes
+
+    from solution import _lib, kernels
+
+    scratch = ctypes.c_size_t(0)
+    path = _lib.load().nf4_linear_path(m, kernels._descs(weights), len(weights), op, xa_rank,
+                                       ctypes.byref(scratch))
+    return path, scratch.value
+
+
 def oracle_w16(packed, qs, dtype="f16"):
     p, st = to_oracle_state(packed, qs)
     w = o.dequantize(p, st, dtype)

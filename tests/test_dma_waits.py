@@ -6,6 +6,12 @@ compiles nf4_gemm.hip for gfx950 to assembly (hipcc cross-compiles without a GPU
 in every forward and input-gradient kernel, that after each group of `buffer_load_dwordx4 ...
 lds` instructions a wait that covers it comes before the next barrier.
 
+The dense kernel of nf4_dense.hip waits by hand-counted groups whose loads stay in flight over
+several barriers, with two wave groups one segment apart.  For it the instruction stream is
+checked to be the counted one (only DMA between the prologue and the last wait, nothing spilled
+to memory), and the schedule itself is replayed in a model of both wave groups: everything read
+has arrived in every wave a barrier before, and nothing is overwritten that may still be read.
+
 A load written as inline assembly is not known to the compiler at all: it neither waits for it
 nor knows that its destination registers are busy until the explicit wait.  A second test
 replays every kernel's instruction stream (each loop body twice, the second pass starting with
@@ -211,6 +217,162 @@ def test_m0_is_settled_before_the_dma_reads_it(gemm_asm, dense_asm):
                 assert not re.match(r"s_\w+ m0\b", before), f"{name}: {before} / {t}"
                 checked += 1
     assert checked > 200
+
+
+def _dense_tokens(body):
+    """[(label or None, [tokens], next labels)] of a kernel's basic blocks, tokens: D (DMA), V
+    (other vector memory), w<n> / W<n> (vmcnt(n) without / with lgkmcnt(0)), B, m."""
+    blocks, label, toks, out = [], None, [], []
+    for t in _strip(body):
+        if t.endswith(":"):
+            blocks.append((label, toks))
+            label, toks = t[:-1], []
+        elif _is_dma(t):
+            toks.append("D")
+        elif re.match(r"(buffer|global|flat|scratch)_", t):
+            toks.append("V")
+        elif t.startswith("s_waitcnt") and "vmcnt(" in t:
+            n = re.search(r"vmcnt\((\d+)\)", t).group(1)
+            toks.append(("W" if "lgkmcnt(0)" in t else "w") + n)
+        elif t.startswith("s_barrier"):
+            toks.append("B")
+        elif "_mfma_" in t:
+            toks.append("m")
+        elif t.startswith(("s_cbranch", "s_branch")):
+            toks.append(("jump" if t.startswith("s_branch") else "maybe") + " " + t.split()[-1])
+        elif t.startswith("s_endpgm"):
+            toks.append("end")
+    return blocks + [(label, toks)]
+
+
+@pytest.mark.timeout(600)
+def test_dense_kernel_issues_what_its_waits_count(dense_asm):
+    from tests.test_skinny_occupancy import _metadata
+
+    meta = dense_asm[dense_asm.index("amdhsa.kernels:"):]
+    names = [n for n in _metadata(dense_asm) if "dense_kernel" in n]
+    assert len(names) == 2
+    for name in names:
+        block = next(b for b in re.split(r"\n  - ", meta) if re.search(rf"\.name:\s+{name}\b", b))
+        for key in ("private_segment_fixed_size", "sgpr_spill_count", "vgpr_spill_count"):
+            assert re.search(rf"\.{key}:\s+(\d+)", block).group(1) == "0", (name, key)
+        blocks = _dense_tokens(dict(_kernels(dense_asm))[name])
+        # the counted runs: a tile's prologue and one step, of 256x256 and of 128x128 tiles
+        grammar = re.compile(r"(D{12}w6B|D{12}w8B|(D{4}W8Bm{16}BD{4}W6Bm{16}B)+|(D{4}W8Bm{8}B)+)$")
+        runs = 0
+        for _, toks in blocks:
+            if "D" not in toks:
+                continue
+            run = [t for t in toks if not t.startswith(("jump", "maybe"))]
+            if run[:12] == ["D"] * 12:  # (waves 4-7 cross one more barrier in a block of their own)
+                run = run[:14]
+            assert grammar.match("".join(run)), (name, toks)
+            runs += 1
+        assert runs >= 6, (name, runs)
+        # from a prologue on, no vector memory but DMA before vmcnt(0), on any way through
+        at = {label: i for i, (label, _) in enumerate(blocks)}
+        todo = [i for i, (_, toks) in enumerate(blocks) if toks[:12] == ["D"] * 12]
+        seen = set()
+        while todo:
+            i = todo.pop()
+            if i in seen:
+                continue
+            seen.add(i)
+            through = True
+            for t in blocks[i][1]:
+                assert t not in ("V", "end"), (name, blocks[i])
+                if t in ("w0", "W0"):
+                    through = False
+                    break
+                if t.startswith(("jump", "maybe")):
+                    todo.append(at[t.split()[1]])
+                    if t.startswith("jump"):
+                        through = False
+                        break
+            if through:
+                todo.append(i + 1)
+
+
+# The schedule of dense_tile (nf4_dense.hip) as one wave group runs it: ("send", half, step),
+# ("read", half, step), ("wait", n) for vmcnt(n) lgkmcnt(0), "barrier".  Halves: w0, w1 (rows p),
+# x0, x1 (rows m); a send is two loads.
+def _dense_schedule(big, steps, group):
+    if big:
+        prologue = [("w0", 0), ("x0", 0), ("x1", 0), ("w1", 0), ("w0", 1), ("x0", 1)]
+        first = 6
+    else:
+        prologue = [(h, u) for u in range(3) for h in ("w0", "x0")]
+        first = 8
+    ops = [("send", h, u) for h, u in prologue] + [("wait", first), "barrier"]
+    ops += ["barrier"] * group
+    for u in range(steps):
+        if big:
+            ops += [("read", h, u) for h in ("x0", "x1", "w0")]
+            ops += [("send", "x1", u + 1), ("send", "w1", u + 1), ("wait", 8), "barrier", "barrier",
+                    ("read", "w1", u), ("send", "w0", u + 2), ("send", "x0", u + 2), ("wait", 6),
+                    "barrier", "barrier"]
+        else:
+            ops += [("read", "x0", u), ("read", "w0", u), ("send", "w0", u + 3),
+                    ("send", "x0", u + 3), ("wait", 8), "barrier", "barrier"]
+    return ops + ["barrier"] * (1 - group) + [("wait", 0), "barrier"]
+
+
+def _dense_hazards(big, steps, schedule=_dense_schedule):
+    """Violations in the schedule of both wave groups, barrier to barrier (what two groups do
+    between the same barriers is unordered)."""
+    stages = 2 if big else 4
+    writes, reads, spans = [], [], []
+    for group in (0, 1):
+        flight, span = [], 0
+        for op in schedule(big, steps, group):
+            if op == "barrier":
+                span += 1
+            elif op[0] == "send":
+                w = [op[1], op[2] % stages, op[2], span, None]  # half, stage, step, issued, arrived
+                writes.append(w)
+                flight += [w, w]
+            elif op[0] == "read":
+                reads.append((op[1], op[2] % stages, op[2], span))
+            else:
+                done = flight[:max(0, len(flight) - op[1])]
+                flight = flight[len(done):]
+                for w in done:
+                    if w not in flight and w[4] is None:
+                        w[4] = span
+        spans.append(span)
+        assert not flight
+    bad = [] if spans[0] == spans[1] else [("barriers", spans)]
+    for half, stage, step, span in reads:
+        for w in writes:
+            if w[:2] != [half, stage]:
+                continue
+            if w[2] == step and not w[4] < span:
+                bad.append(("read before it arrived", half, step, span, w))
+            if w[2] > step and not w[3] > span:
+                bad.append(("overwritten while it may be read", half, step, span, w))
+        assert sum(w[:3] == [half, stage, step] for w in writes) == 2  # both groups' shares
+    return bad
+
+
+@pytest.mark.parametrize("big", [True, False])
+def test_dense_schedule_reads_what_arrived(big):
+    for steps in range(1, 14):
+        assert not _dense_hazards(big, steps), steps
+
+
+def test_dense_schedule_model_flags_a_missing_wait_and_an_early_send():
+    def later_wait(big, steps, group):
+        return [("wait", 10) if op == ("wait", 6) else op
+                for op in _dense_schedule(big, steps, group)]
+
+    def early_send(big, steps, group):  # x0 two steps ahead while this step's is being read
+        swap = {"x1": ("x0", 1), "x0": ("x1", -1)}
+        ops, first = _dense_schedule(big, steps, group), 6
+        return ops[:first] + [("send", swap[op[1]][0], op[2] + swap[op[1]][1])
+                              if op[0] == "send" and op[1] in swap else op for op in ops[first:]]
+
+    assert any("arrived" in b[0] for b in _dense_hazards(True, 5, later_wait))
+    assert any("overwritten" in b[0] for b in _dense_hazards(True, 5, early_send))
 
 
 def test_replay_model_flags_a_register_used_before_its_wait():

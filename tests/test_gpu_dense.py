@@ -7,7 +7,7 @@ the dequantized weight and, with one-hot rows, against the weight bit for bit.""
 import pytest
 import torch
 
-from tests.gpu_util import assert_rel, banner, random_weight
+from tests.gpu_util import OP_DX, PATH_DENSE, assert_rel, banner, linear_path, random_weight
 
 pytestmark = pytest.mark.gpu
 
@@ -135,3 +135,64 @@ def test_dense_forward_keeps_non_finite_lora_to_its_segment(cuda, dtype, rows, k
         rest = torch.ones(m, dtype=torch.bool, device=cuda)
         rest[5] = rest[m - 1] = False
         assert torch.equal(y_bad[rest], y[rest])
+
+
+def _mixed(rows, k, dev):
+    """Segments of different formats: nested absmax with blocks of 64, fp32 absmax with blocks of
+    128, nested with blocks of 256."""
+    kinds = [(64, True), (128, False), (256, True)]
+    return [random_weight(n, k, seed=340 + i, dev=dev, blocksize=kinds[i % 3][0], nested=kinds[i % 3][1])
+            for i, n in enumerate(rows)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,m", [([520, 200, 576], 3072, 1300), ([520, 200, 576], 3072, 3001),
+                                      ([776, 520], 2048, 4100)])
+def test_dense_forward_mixed_weights_and_slabs(cuda, dtype, rows, k, m):
+    """Segments of three weight formats and an adapter on the first and on the last one, their
+    edges inside tiles."""
+    from solution import kernels
+
+    banner("dense fwd mixed", dtype, rows, k, m)
+    weights = _mixed(rows, k, cuda)
+    assert linear_path(weights, m)[0] == PATH_DENSE
+    w = kernels.dequant(weights, dtype)
+    n = sum(rows)
+    g = torch.Generator(device=cuda).manual_seed(11)
+    x = torch.randn(m, k, generator=g, device=cuda).to(dtype)
+    bias = torch.randn(n, generator=g, device=cuda).to(dtype)
+    ref, loras = x.float() @ w.float().T + bias.float(), []
+    for seg, r, lo in ((0, 16, 0), (len(rows) - 1, 40, n - rows[-1])):
+        t, b = _lora(m, r, k, rows[seg], dtype, cuda, 12 + seg)
+        loras.append(kernels.make_lora(seg, r, 0.5, t=t, b=b))
+        ref[:, lo:lo + rows[seg]] += 0.5 * t.float() @ b.float().T
+    assert_rel(kernels.linear_fwd(x, weights, bias, loras), ref, what="y")
+    idx = (torch.arange(m, device=cuda) * 61 + 7) % k
+    hot = torch.zeros(m, k, dtype=dtype, device=cuda)
+    hot[torch.arange(m, device=cuda), idx] = 1
+    assert torch.equal(kernels.linear_fwd(hot, weights), w.T[idx])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,m", [([1536, 256, 320], 1536, 1025), ([3008, 64, 128], 1536, 3001)])
+def test_dense_input_gradient_mixed_weights_and_slabs(cuda, dtype, rows, k, m):
+    from solution import kernels
+
+    banner("dense dx mixed", dtype, rows, k, m)
+    weights = _mixed(rows, k, cuda)
+    assert linear_path(weights, m, OP_DX)[0] == PATH_DENSE
+    w = kernels.dequant(weights, dtype)
+    n = sum(rows)
+    g = torch.Generator(device=cuda).manual_seed(13)
+    dy = torch.randn(m, n, generator=g, device=cuda).to(dtype)
+    ref, loras = dy.float() @ w.float(), []
+    for seg, r in ((0, 16), (2, 40)):
+        da, at = _lora(m, r, n, k, dtype, cuda, 14 + seg)
+        a = at.T.contiguous()
+        loras.append(kernels.make_lora(seg, r, 2.0, a=a, da=da))
+        ref += da.float() @ a.float()
+    assert_rel(kernels.linear_dx(dy, weights, loras), ref, what="dx")
+    idx = (torch.arange(m, device=cuda) * 61 + 7) % n
+    hot = torch.zeros(m, n, dtype=dtype, device=cuda)
+    hot[torch.arange(m, device=cuda), idx] = 1
+    assert torch.equal(kernels.linear_dx(hot, weights), w[idx])

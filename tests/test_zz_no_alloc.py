@@ -7,7 +7,8 @@ where the array forces a smaller split."""
 import pytest
 import torch
 
-from tests.gpu_util import assert_rel, banner, random_weight
+from tests.gpu_util import (OP_DX, OP_DX_NOALLOC, PATH_DENSE, assert_rel, banner, linear_path,
+                            random_weight)
 
 pytestmark = pytest.mark.gpu
 
@@ -77,17 +78,6 @@ QKV_15B = [(1536, 1536), (256, 1536), (256, 1536)]
 QKV_7B = [(3584, 3584), (512, 3584), (512, 3584)]
 
 
-def _path(weights, m, op):
-    import ctypes
-
-    from solution import _lib, kernels
-
-    scratch = ctypes.c_size_t(0)
-    path = _lib.load().nf4_linear_path(m, kernels._descs(weights), len(weights), op, 0,
-                                       ctypes.byref(scratch))
-    return path, scratch.value
-
-
 def _problem(shapes, m, seed, dtype, dev):
     weights = [random_weight(n, k, seed=seed + i, dev=dev) for i, (n, k) in enumerate(shapes)]
     g = torch.Generator(device=dev).manual_seed(seed)
@@ -104,7 +94,8 @@ def test_noalloc_on_the_dense_route_matches_linear_dx(cuda, dtype, shapes, m):
 
     banner("noalloc dense", dtype, shapes, m)
     weights, dy = _problem(shapes, m, 900, dtype, cuda)
-    assert _path(weights, m, 1) == _path(weights, m, 2) and _path(weights, m, 2)[0] == 6
+    path = linear_path(weights, m, OP_DX_NOALLOC)
+    assert path[0] == PATH_DENSE and path == linear_path(weights, m, OP_DX)
     ref = kernels.linear_dx(dy, weights)
     out = _noalloc(dy, weights, torch.full_like(ref, float("nan")))
     assert torch.equal(out, ref)
@@ -119,7 +110,7 @@ def test_noalloc_without_scratch_is_the_fused_product(cuda, dtype, shapes, m):
 
     banner("noalloc unsplit", dtype, shapes, m)
     weights, dy = _problem(shapes, m, 910, dtype, cuda)
-    assert _path(weights, m, 1)[0] == 6
+    assert linear_path(weights, m, OP_DX)[0] == PATH_DENSE
     ref = torch.empty(m, shapes[0][1], dtype=dtype, device=cuda)
     _lib.check(_lib.load().nf4_linear_dx(
         dy.data_ptr(), m, dy.stride(0), kernels._descs(weights), len(weights), None, 0,
@@ -133,7 +124,7 @@ def test_noalloc_calls_without_scratch_overlap(cuda):
     """Two streams, two problems of a size that needs no scratch, several calls each in flight."""
     m = 1025
     problems = [_problem(QKV_15B, m, 920 + 10 * i, torch.float16, cuda) for i in range(2)]
-    assert _path(problems[0][0], m, 2)[1] == 0
+    assert linear_path(problems[0][0], m, OP_DX_NOALLOC)[1] == 0
     banner("noalloc overlapping", QKV_15B, m)
     outs = [[torch.full((m, 1536), float("nan"), dtype=torch.float16, device=cuda)
              for _ in range(8)] for _ in problems]
