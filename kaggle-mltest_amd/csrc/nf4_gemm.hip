@@ -3515,6 +3515,9 @@ int launch_dense(GemmArgs &g, const DenseRoute &r, int nw, bool dx, void *worksp
 extern "C" size_t nf4_linear_fwd_workspace(int64_t m, const nf4_weight *ws, int nw, int dtype) {
     (void)dtype;
     if (!ws || nw < 1 || nw > kMaxSeg || m <= 0) return 0;
+    int64_t n = 0;
+    for (int i = 0; i < nw; ++i) n += ws[i].rows;
+    if (n == 0 || ws[0].cols == 0) return 0;  // (the plans of few tokens divide by both)
     const Plan p = plan_fwd(m, ws, nw);
     const DenseRoute dense = dense_route_fwd(m, ws, nw, p);
     // (the partials also where the dense route is taken: a call that it does not fit)
@@ -3589,6 +3592,7 @@ extern "C" int nf4_linear_fwd_tiled(const void *x, int64_t m, int64_t ldx, const
         if (l.a) xa_rank = l.rank > xa_rank ? l.rank : xa_rank;
     }
     if (m == 0 || n_out == 0) return NF4_OK;
+    if (g.K == 0 && m <= kSkinnyMaxM && tile < 0) return NF4_ERR_UNSUPPORTED;  // (its plans divide by K)
     g.bias = static_cast<const uint16_t *>(bias);
     g.out = y;
     g.ld_out = ldy;

@@ -91,3 +91,29 @@ def test_noalloc_shares_its_array_only_where_its_fused_plan_would(lib):
             seen.add((p, q, noalloc > 0))
     assert {(DENSE, TILED, False), (DENSE, DENSE, True), (TILED, TILED, False),
             (TILED, TILED, True)} <= seen
+
+
+@pytest.mark.parametrize("k", [0, 64, 192, 256, 4096])
+@pytest.mark.parametrize("rows", [(0,), (0, 0), (0, 96)])
+def test_queries_answer_for_empty_weights(lib, rows, k):
+    """No rows or no columns: nothing to launch, and nothing to divide by either."""
+    shapes = [(r, k) for r in rows]
+    ws = _weights(shapes)
+    for m in (1, 2, 3, 16, 17, 20, 32, 33, 64, 65, 600, 3000):
+        empty = sum(rows) == 0 or k == 0
+        for op in (FWD, DX, DX_NOALLOC):
+            p, used, query = path(lib, shapes, m, op)
+            assert used <= max(query, STATIC_SCRATCH if op == DX_NOALLOC else 0)
+            if empty:
+                assert p == -1 and (op == DX or query == 0)
+
+
+def test_an_empty_reduction_of_few_tokens_is_refused(lib):
+    """K = 0 with rows to write: refused before any launch."""
+    from solution._lib import NF4_ERR_UNSUPPORTED
+
+    buf = (ctypes.c_uint16 * 4096)()
+    at = ctypes.addressof(buf) + 255 & ~255
+    for m in (1, 3, 20, 64):
+        assert lib.nf4_linear_fwd(at, m, 8, _weights([(32, 0)]), 1, None, None, 0, at, 32, 0, None,
+                                  0, None) == NF4_ERR_UNSUPPORTED
