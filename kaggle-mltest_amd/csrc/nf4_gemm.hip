@@ -2917,7 +2917,7 @@ Plan make_plan(int64_t m, int64_t big, int64_t small, int64_t steps, int max_spl
     return sl.plan;
 }
 
-Plan plan_gemv(int64_t m, const nf4_weight *ws, int nw) {
+Plan plan_gemv(int64_t m, const nf4_weight *ws, int nw, int max_splits = kMaxSplits) {
     int64_t tiles = 0;
     for (int i = 0; i < nw; ++i) tiles += (ws[i].rows + 31) / 32;
     const int64_t steps = ws[0].cols / BR;
@@ -2930,7 +2930,7 @@ Plan plan_gemv(int64_t m, const nf4_weight *ws, int nw) {
         splits = kCUs / tiles;
         const int64_t by_steps = steps / (2 * waves);
         if (splits > by_steps) splits = by_steps;
-        if (splits > kMaxSplits) splits = kMaxSplits;
+        if (splits > max_splits) splits = max_splits;
         if (splits < 1) splits = 1;
         while (splits > 1 && (splits - 1) * ((steps + splits - 1) / splits) >= steps) --splits;
     }
@@ -3180,7 +3180,9 @@ Plan plan_fwd(int64_t m, const nf4_weight *ws, int nw, int tile = -1, int splits
         return t32 < 0.95 * t ? p32 : p;
     }
     if (tile < 0 && m <= kDecodeMaxM && ws[0].cols % DK == 0) return plan_decode(ws, nw);
-    if (tile < 0 && m <= kGemvMaxM) return plan_gemv(m, ws, nw);
+    // (not split where only the LoRA operands' alignment kept the row-streaming path from it: the
+    // workspace query has not seen them)
+    if (tile < 0 && m <= kGemvMaxM) return plan_gemv(m, ws, nw, rows_ok(m, ws, nw) ? 1 : kMaxSplits);
     int64_t big = 0, small = 0;
     for (int i = 0; i < nw; ++i) {
         big += (ws[i].rows + 255) / 256;

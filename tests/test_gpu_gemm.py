@@ -366,6 +366,25 @@ def test_lora_xa_decode_sizes(cuda, dtype, m, k, r):
         assert_rel(t[i], ref, what=f"xa {i}")
 
 
+@pytest.mark.parametrize("m", [1, 2])
+def test_decode_with_a_lora_operand_off_dword_alignment(cuda, m):
+    """LoRA B two bytes off: the row-streaming path does not take it, and the small-M kernel that
+    does needs no more workspace than the query, which does not see adapters, returned."""
+    from solution import kernels
+
+    rows, k, r = 512, 18496, 16
+    banner("lora off alignment", m, rows, k)
+    w = random_weight(rows, k, 61, cuda)
+    x = _x(m, k, 62, cuda)
+    g = torch.Generator().manual_seed(63)
+    t = torch.randn(m, r, generator=g).half().to(cuda)
+    b = torch.empty(rows * r + 1, dtype=torch.float16, device=cuda)[1:].view(rows, r)
+    b.copy_(torch.randn(rows, r, generator=g) * 0.05)
+    y = kernels.linear_fwd(x, [w], None, [kernels.make_lora(0, r, 0.5, t=t, b=b)])
+    ref = x.float() @ kernels.dequant([w]).float().T + 0.5 * t.float() @ b.float().T
+    assert_rel(y, ref, what="y")
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("m,k,r", [(1, 8, 16), (3, 4104, 16), (17, 2048, 5), (33, 6152, 8), (63, 8960, 16)])
 def test_lora_xa_decode_step_edges(cuda, dtype, m, k, r):
