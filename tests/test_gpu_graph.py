@@ -39,3 +39,34 @@ def test_stack_graph_replays_match_eager(cuda, m):
         for i, (a, b) in enumerate(zip(got, ref)):
             assert torch.equal(a, b), f"replay {rep}, output {i}"
     assert other is st.per_layer[1]
+
+
+def test_dense_calls_replay_in_a_graph(cuda):
+    """The dense route captured (its workspaces from the graph's pool, unsplit and with a split
+    reduction): every replay gives the eager result, with eager calls of the same route between."""
+    from solution import kernels
+    from tests.gpu_util import OP_DX, PATH_DENSE, linear_path, random_weight
+
+    banner("graph replay dense")
+    g = torch.Generator(device=cuda).manual_seed(31)
+    calls = []
+    for rows, k, m, dx in (([520, 776], 3072, 1300, False), ([520, 776], 3072, 3001, False),
+                           ([1536, 256, 256], 1536, 1025, True), ([3008, 64], 1536, 3001, True)):
+        w = [random_weight(n, k, seed=350 + i, dev=cuda) for i, n in enumerate(rows)]
+        assert linear_path(w, m, OP_DX if dx else 0)[0] == PATH_DENSE
+        x = torch.randn(m, sum(rows) if dx else k, generator=g, device=cuda).half()
+        calls.append((kernels.linear_dx if dx else kernels.linear_fwd, x, w))
+    ref = [f(x, w) for f, x, w in calls]
+    out = [torch.empty_like(r) for r in ref]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for (f, x, w), o in zip(calls, out):
+            f(x, w, out=o)
+    for rep in range(3):
+        for o in out:
+            o.fill_(float("nan"))
+        eager = [f(x, w) for f, x, w in calls]
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (a, b, c) in enumerate(zip(out, ref, eager)):
+            assert torch.equal(a, b) and torch.equal(c, b), f"replay {rep}, call {i}"
