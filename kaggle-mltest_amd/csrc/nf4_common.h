@@ -345,6 +345,27 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
                                       c, false);
 }
 
+// 32x32x16 MFMA on fp16 or bf16 fragments.
+template <int DT>
+__device__ __forceinline__ float16_t mfma32(const u32x4_t &a, const u32x4_t &b, const float16_t &c) {
+    if constexpr (DT == NF4_BF16) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf168_t, a),
+                                                      __builtin_bit_cast(bf168_t, b), c, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a),
+                                                     __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+    }
+}
+
+// A value known to be the same in every lane, kept in scalar registers (the compiler otherwise
+// can lose track through VALU-computed integer division and then wraps every buffer load that
+// uses it in a per-lane loop).
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32));
+    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 // ----------------------------------------------------------------- buffer resources
 //
 // Main-loop loads go through buffer resources: an offset at or past the resource's byte range

@@ -14,25 +14,9 @@ constexpr int HALF = 128 * 128;  // bytes of one staged half tile: 128 rows x 64
 constexpr int kLds = 8 * HALF;   // 128 KB: two steps of a 256x256 tile, four of a 128x128 tile
 
 template <int DT>
-__device__ __forceinline__ float16_t mfma32d(const u32x4_t &a, const u32x4_t &b, const float16_t &c) {
-    if constexpr (DT == NF4_BF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf168_t, a),
-                                                      __builtin_bit_cast(bf168_t, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a),
-                                                     __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
-}
-
-template <int DT>
 __device__ __forceinline__ float widen(uint32_t v) {
     if constexpr (DT == NF4_BF16) return __uint_as_float(v << 16);
     else return static_cast<float>(__builtin_bit_cast(half_t, static_cast<uint16_t>(v)));
-}
-
-__device__ __forceinline__ int64_t uniform(int64_t v) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32));
-    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 // Values 0 .. 7 (zero from `lim` on) of a LoRA row, `step` elements apart.
@@ -139,7 +123,7 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
 #pragma unroll
             for (int g = 0; g < HM; ++g)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) c[g][i] = mfma32d<DT>(fw[i][ks], fx[g][ks], c[g][i]);
+                for (int i = 0; i < 2; ++i) c[g][i] = mfma32<DT>(fw[i][ks], fx[g][ks], c[g][i]);
     };
 
     // A segment ends with this wave's fragment reads complete (so the next segment's DMA of
@@ -228,7 +212,7 @@ __device__ __forceinline__ void dense_tile(const DenseArgs &a, uint8_t *lds, int
                     for (int g = 0; g < HM; ++g) {
                         const u32x4_t ft = *reinterpret_cast<const u32x4_t *>(
                             lds + 256 * 32 + (g * 128 + wm * 32 + r32) * 32 + kh * 16);
-                        const float16_t v = sl.scale * mfma32d<DT>(fl, ft, (float16_t){});
+                        const float16_t v = sl.scale * mfma32<DT>(fl, ft, (float16_t){});
 #pragma unroll
                         for (int e = 0; e < 16; ++e)
                             acc[h][g][i][e] += __uint_as_float(__float_as_uint(v[e]) & mask[e / 4][e % 4]);
@@ -332,8 +316,8 @@ __device__ __forceinline__ void band_tile(uint32_t t, uint32_t pt, uint32_t mt, 
     const uint32_t bands = mt < 8 ? 1 : (mt + 2) / 5;
     const uint32_t band = ((t / pt + 1) * bands - 1) / mt;
     const uint32_t lo = band * mt / bands, hi = (band + 1) * mt / bands, r = t - lo * pt;
-    p = uniform(r / (hi - lo));
-    m = uniform(lo + r % (hi - lo));
+    p = uniform64(r / (hi - lo));
+    m = uniform64(lo + r % (hi - lo));
 }
 
 // Workgroups [0, blocks0) run 256x256 tiles (of a split plan each over its share of the
@@ -410,7 +394,7 @@ __global__ __launch_bounds__(256) void dequant_strips_kernel(const StripArgs a) 
     __shared__ __attribute__((aligned(16))) uint8_t tile[128 * 256];
     __shared__ float s_code2[256];
     const uint32_t nt = static_cast<uint32_t>(a.tile0[a.nseg]);
-    const int64_t ti = uniform(blockIdx.x % nt), k0 = uniform(int64_t(blockIdx.x / nt) * 128);
+    const int64_t ti = uniform64(blockIdx.x % nt), k0 = uniform64(int64_t(blockIdx.x / nt) * 128);
     int seg = 0;
 #pragma unroll
     for (int i = 1; i < NF4_MAX_SEGMENTS; ++i)

@@ -109,17 +109,6 @@ struct GemmArgs {
     int rows_parts;               // row-streaming path: K parts per row
 };
 
-template <int DT>
-__device__ __forceinline__ float16_t mfma32(const u32x4_t &a, const u32x4_t &b, const float16_t &c) {
-    if constexpr (DT == NF4_BF16) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf168_t, a),
-                                                      __builtin_bit_cast(bf168_t, b), c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a),
-                                                     __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
-    }
-}
-
 // 16x16x32 MFMA: lane l holds row (A) / column (B) l % 16, k = 8 (l / 16) .. + 7; D lane l
 // holds rows 4 (l / 16) .. + 3 of column l % 16.
 template <int DT>
@@ -158,15 +147,6 @@ __device__ __forceinline__ int seg_of_step(const GemmArgs &a, int64_t t) {
     for (int i = 1; i < kMaxSeg; ++i)
         if (i < a.nseg && t >= a.step_start[i]) s = i;
     return s;
-}
-
-// A value known to be the same in every lane, kept in scalar registers (the compiler otherwise
-// can lose track through VALU-computed integer division and then wraps every buffer load that
-// uses it in a per-lane loop).
-__device__ __forceinline__ int64_t uniform64(int64_t v) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32));
-    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 // Tiles run m fastest: the dispatcher deals workgroups to the 8 XCDs in turn (XCD = id mod 8,
