@@ -5,11 +5,11 @@
  * backward, on one AMD Instinct MI355X.  Every entry point takes plain device pointers, sizes, a
  * dtype code and a HIP stream (as void*), launches asynchronously on that stream and returns an
  * int status (NF4_OK == 0).  The caller allocates every output and workspace, and apart from
- * one entry point the library owns no device memory and keeps no state between calls, so it is
- * reentrant and thread-safe.  The exception is nf4_linear_dx_noalloc (for callers that cannot
- * allocate): its workspace is a 64 MiB device array that the library holds on every
- * GPU it runs on until the process ends, and calls of it that use that array and overlap on one
- * GPU race.
+ * one entry point the library owns no device memory; between calls it keeps only host-side plans
+ * (a small table per thread, of sizes and no pointers), so it is reentrant and thread-safe.  The
+ * exception is nf4_linear_dx_noalloc (for callers that cannot allocate): its workspace is a
+ * 64 MiB device array that the library holds on every GPU it runs on until the process ends, and
+ * calls of it that use that array and overlap on one GPU race.
  *
  * Weight format (bitsandbytes 0.50.2 QuantState, as read by the reference at
  * /root/reference/solution/nf4.py:46-53,112-131):

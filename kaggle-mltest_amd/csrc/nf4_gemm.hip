@@ -1829,8 +1829,8 @@ __global__ __launch_bounds__(RT * KP * 64) void skinny_kernel(const GemmArgs a) 
 // the activations staged in it).  Bound by VALU + MFMA issue: on the 16-row kernel the 7B
 // gate|up at M = 64 issued 5.85 VALU instructions per element (a table per 32 elements, the
 // activations staged again for every 128 rows) and read four fragments per A fragment; here 4.0 and two.
-// A workgroup of 5 x 2 waves owns 160 rows: the 1184 row tiles of the 7B gate|up are 237
-// workgroups, one round of the chip, where 128-row workgroups took two with a split
+// A workgroup of 5 x 2 waves owns 160 rows: the 7B gate|up pair is 238 workgroups (119 per
+// segment), one round of the chip, where 128-row workgroups took two with a split
 // reduction.  That product at M = 64: 61 -> 46 us, at 32: 44 -> 38.  (Before the fragments were read
 // ahead 50 us; then three k-parts, 15 waves, 50.6, four or two row tiles, or a split
 // reduction, 61 us and more.)
@@ -3130,7 +3130,10 @@ bool skinny_ok(int64_t m, const nf4_weight *ws, int nw, int xa_rank) {
 }
 
 // The 32-row skinny plan and its time: rounds of 160-row workgroups over the CUs, each step of
-// its two k-parts 2.85 us at 33-64 tokens and 2.3 at 17-32 (7B gate|up: 45.8 and 38.2 us).
+// its two k-parts 2.85 us at 33-64 tokens and 2.3 at 17-32.  The two step times are those of one
+// product (7B gate|up: 45.8 and 38.2 us) with the 6 us beside them assumed, and nothing stands for
+// the activations read or for a round that is partly full: the margin of 5 % against the 16-row
+// plan below keeps it to about 32900-41000 stacked rows and, at some K and M, 65700-82000.
 Plan plan_skinny32(int64_t m, const nf4_weight *ws, int nw, double *cost) {
     int64_t wgs = 0;
     for (int i = 0; i < nw; ++i) wgs += (ws[i].rows + 32 * kTallRt - 1) / (32 * kTallRt);
@@ -3404,8 +3407,9 @@ double fused_time(const Plan &p, int64_t small_tiles, int extra_segs) {
 }
 
 // Taken where it is 4 % faster by the two models (10 % with a split reduction, whose partials
-// come on top of the weight in the workspace): of 308 measured (projection, direction, M, dtype)
-// points no fused one faster by more than 1 % is given up.  Below 512 tokens the
+// come on top of the weight in the workspace).  Both routes timed at the 162 of 416 (Qwen2.5-1.5B
+// and -7B projection, direction, dtype, M = 512 .. 8192) where it is taken: 0.62 to 1.017 of the
+// fused time, above 1.003 at one (1.5B o forward, fp16, M = 3072: 35.3 against 34.7 us).  Below 512 tokens the
 // dequantization alone costs what the fused kernels need; from 2^23 on the dense kernel's 32-bit
 // tile arithmetic (band_tile: token tiles squared / 5) would come near its end.
 DenseRoute dense_route(int64_t P, int64_t m, int64_t R, double dequant_us, double fused_us) {

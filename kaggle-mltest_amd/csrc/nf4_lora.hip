@@ -198,10 +198,12 @@ __global__ __launch_bounds__(256) void rowvec_kernel(const Jobs jobs, int64_t m_
     float acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
-    // Latency-bound: all loads of up to two 2048-wide steps are issued before the first product
-    // (two adapters, 64 tokens, K = 3584: 9.1 -> 4.8 us; with a branch per token every load was
-    // waited for before the next was issued).  So no branch around a load: tokens past the last
-    // one load it again (never stored), lanes past k load the row's start and keep their sum.
+    // Latency-bound, so no branch around a load: with one per token every load was waited for
+    // before the next was issued (two adapters, 64 tokens, K = 3584: 9.1 -> 4.8 us without).
+    // Tokens past the last one load it again (never stored), lanes past k load the row's start
+    // and keep their sum.  Two 2048-wide steps at a time: up to 4 tokens all their loads are
+    // issued before the first product; with 8 the compiler issues one step's nine loads together
+    // and the second step's after about 30 of the first's products (73 VGPRs).
     auto steps = [&](int64_t kb, auto n) {
         constexpr int N = decltype(n)::value;
         u32x4_t a[N], x[N][MT];

@@ -33,7 +33,12 @@ INT8_FORWARD = False
 
 
 # Token count from which the gate|up GEMM carries the SwiGLU epilogue (its tiles are the large
-# forward tiles; the decode-size GEMM paths keep the separate SwiGLU step).
+# forward tiles; the decode-size GEMM paths keep the separate SwiGLU step).  The epilogue exists on
+# the fused dequant-GEMM only, while the plain product of large batches may take the dense route:
+# fused against separate, the forward is 74 / 85 us at 1000 tokens, 133 / 148 at 2048 and 477 / 534
+# at 8192 (1.5B, bf16), 559 / 577 at 2048 and 2130 / 2003 at 8192 (7B); the backward's recomputation
+# 85 / 88, 156 / 154 and 576 / 561 (1.5B), 619 / 600 and 2329 / 2070 (7B).  So the backward from
+# about 1500 tokens and the 7B forward at 8192 would be faster separate; the rule has no such bound.
 FUSED_MIN_TOKENS = 65
 
 

@@ -5,13 +5,14 @@ Mirror of /root/reference/solution/nf4.py: the same names and signatures (`dequa
 `_gemm_dtype`, `_base_uses_fused_kernel_for`), the same routing rules, and the same fall-back to
 bitsandbytes' original function for anything this path does not cover.  Underneath, the
 reference's Triton dequant + cuBLAS GEMM becomes one fused dequant-GEMM launch
-(`nf4_linear_fwd` / `nf4_linear_dx` in libnf4_mi355x.so): the fp16 weight is never written
-to HBM.
+(`nf4_linear_fwd` / `nf4_linear_dx` in libnf4_mi355x.so), which does not write the fp16 weight to
+HBM, except for large products from 512 tokens on where one dequantization into a workspace and a
+plain 16-bit GEMM are faster.
 
 Differences from the reference, by design:
 * the double-quantized absmax is rebuilt inside the kernels from the uint8 codes (no cached
   fp32 absmax, nf4.py:41-55), bit for bit the same value;
-* fp16 and bf16 GEMMs are one fused launch; an fp32 GEMM (the reference's path when neither
+* fp16 and bf16 GEMMs are one fused call; an fp32 GEMM (the reference's path when neither
   autocast nor a half compute dtype is set) dequantizes to fp32 with the HIP kernel and
   multiplies with torch's fp32 GEMM, as the reference's NF4Linear does in fp32;
 * a library that cannot be loaded, or an error status from it, sends the call to
