@@ -3159,7 +3159,7 @@ Plan plan_fwd(int64_t m, const nf4_weight *ws, int nw, int tile = -1, int splits
         // need it, p is the plan without adapters, and so is its time, to the last bit: with the
         // launch on both sides of the 0.95 the choice would hang on the adapters.
         if (xa_rank > 0 && skinny_fx_ok(p, xa_rank)) t32 += xa_launch_cost(ws[0].cols);
-        else plan_skinny(m, ws, nw, &t);
+        else if (xa_rank > 0) plan_skinny(m, ws, nw, &t);
         return t32 < 0.95 * t ? p32 : p;
     }
     if (tile < 0 && m <= kDecodeMaxM && ws[0].cols % DK == 0) return plan_decode(ws, nw);
